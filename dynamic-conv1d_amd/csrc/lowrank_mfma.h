@@ -280,6 +280,15 @@ __device__ __forceinline__ F pick(const S (&a)[kMaxGroups], int g, F S::*f) {
   return g == 0 ? a[0].*f : g == 1 ? a[1].*f : g == 2 ? a[2].*f : a[3].*f;
 }
 
+// The argument block of a kernel whose only parameter is an A, as the scalar
+// unit reads it: a field at a uniform run-time index (a group's pointers) is one
+// scalar load, where indexing the by-value parameter would copy it to scratch
+// and pick()'s selects compile to a tree of branches with a load in each.
+template <class A>
+__device__ __forceinline__ const __attribute__((address_space(4))) A* kernel_args() {
+  return (const __attribute__((address_space(4))) A*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
 // Longest run (16-row tiles) of the MFMA forward / backward for p whose rows
 // fit the buffer resources (0: not even one tile; the generic kernels take p).
 int64_t lr_fwd_max_run_tiles(const LrProblem& p);
