@@ -289,6 +289,11 @@ __device__ __forceinline__ const __attribute__((address_space(4))) A* kernel_arg
   return (const __attribute__((address_space(4))) A*)__builtin_amdgcn_kernarg_segment_ptr();
 }
 
+// 16 bytes of global memory (a pointer read from kernel_args is generic to the compiler).
+__device__ __forceinline__ u32x4 gload128(const void* p) {
+  return *(const __attribute__((address_space(1))) u32x4*)(reinterpret_cast<uintptr_t>(p));
+}
+
 // Longest run (16-row tiles) of the MFMA forward / backward for p whose rows
 // fit the buffer resources (0: not even one tile; the generic kernels take p).
 int64_t lr_fwd_max_run_tiles(const LrProblem& p);

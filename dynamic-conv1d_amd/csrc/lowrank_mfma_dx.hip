@@ -35,11 +35,12 @@ __global__ __launch_bounds__(64 * fwd_wg_waves(W, RC)) void lr_dx_mfma(LrArgs a)
   const int lb0 = xcd_remap(blockIdx.x, a.nblk);
   const int g = __builtin_amdgcn_readfirstlane(lb0 / a.nblk1);
   const int lb = lb0 - g * a.nblk1;
-  const uint16_t* __restrict__ dy = reinterpret_cast<const uint16_t*>(pick(a.grp, g, &LrFwdGroup::x));
-  const uint16_t* __restrict__ z = reinterpret_cast<const uint16_t*>(pick(a.grp, g, &LrFwdGroup::z));
-  const uint16_t* __restrict__ U = reinterpret_cast<const uint16_t*>(pick(a.grp, g, &LrFwdGroup::U));
-  const uint16_t* __restrict__ sw = reinterpret_cast<const uint16_t*>(pick(a.grp, g, &LrFwdGroup::sw));
-  uint16_t* __restrict__ dx = reinterpret_cast<uint16_t*>(pick(a.grp, g, &LrFwdGroup::y));
+  const auto* gp = kernel_args<LrArgs>()->grp + g;  // the group's pointers: scalar loads at a uniform offset
+  const uint16_t* __restrict__ dy = reinterpret_cast<const uint16_t*>(gp->x);
+  const uint16_t* __restrict__ z = reinterpret_cast<const uint16_t*>(gp->z);
+  const uint16_t* __restrict__ U = reinterpret_cast<const uint16_t*>(gp->U);
+  const uint16_t* __restrict__ sw = reinterpret_cast<const uint16_t*>(gp->sw);
+  uint16_t* __restrict__ dx = reinterpret_cast<uint16_t*>(gp->y);
   const int chunk = lb % a.nch, sgp = lb / a.nch;
   const int D = a.D, Tn = a.Tn, R = a.R, RK = a.RK;
   const int dl = chunk * 128 + 8 * n;  // first channel of the lane's octet

@@ -75,23 +75,33 @@ template <int W, int RC>
 __device__ __forceinline__ void stage_u(u32x2* __restrict__ lds, const uint16_t* __restrict__ U,
                                         const uint16_t* __restrict__ sw, int R, int RK, int D, int64_t WD, int dl,
                                         bool chv, int q, int lane, int wave) {
+  // Loads without branches, a chunk's four in flight together: a lane past D or a
+  // row past RK reads the first piece of U (of static_w in a pass of the static
+  // rank alone), which exists and is 16-byte aligned, and drops it.
+  const uint16_t* const safe = R > 0 ? U : sw;
   for (int kc = wave; kc < W * RC; kc += fwd_wg_waves(W, RC)) {
     const int k = kc / RC, c = kc - k * RC;
     u32x4 rows[4];
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const int r = 16 * c + 4 * q + kk;
-      const uint16_t* src = nullptr;
-      if (chv && r < R) src = U + (int64_t)r * WD + (int64_t)k * D + dl;
-      else if (chv && r < RK) src = sw + (int64_t)k * D + dl;
-      rows[kk] = src ? *reinterpret_cast<const u32x4*>(src) : u32x4{0u, 0u, 0u, 0u};
+      const int64_t at = (int64_t)k * D + dl;
+      const uint16_t* src = r < R ? U + r * WD + at : sw + at;
+      src = chv && r < RK ? src : safe;
+      rows[kk] = gload128(src);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const bool ok = chv && 16 * c + 4 * q + kk < RK;
+#pragma unroll
+      for (int h = 0; h < 4; ++h) rows[kk][h] = ok ? rows[kk][h] : 0u;
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      u32x2 v;
-      v[0] = elem16(rows[0], j) | (elem16(rows[1], j) << 16);
-      v[1] = elem16(rows[2], j) | (elem16(rows[3], j) << 16);
-      lds[(kc * 8 + j) * 64 + lane] = v;
+      // v_perm: the even (odd) channels' halves of two rows
+      const uint32_t hl = j & 1 ? 0x07060302u : 0x05040100u;
+      lds[(kc * 8 + j) * 64 + lane] = u32x2{__builtin_amdgcn_perm(rows[1][j >> 1], rows[0][j >> 1], hl),
+                                            __builtin_amdgcn_perm(rows[3][j >> 1], rows[2][j >> 1], hl)};
     }
   }
 }
@@ -130,11 +140,12 @@ void lr_fwd_mfma(LrArgs a) {
   const int lb0 = xcd_remap(blockIdx.x, a.nblk);
   const int g = __builtin_amdgcn_readfirstlane(lb0 / a.nblk1);
   const int lb = lb0 - g * a.nblk1;
-  const uint16_t* __restrict__ x = reinterpret_cast<const uint16_t*>(pick(a.grp, g, &LrFwdGroup::x));
-  const uint16_t* __restrict__ z = reinterpret_cast<const uint16_t*>(pick(a.grp, g, &LrFwdGroup::z));
-  const uint16_t* __restrict__ U = reinterpret_cast<const uint16_t*>(pick(a.grp, g, &LrFwdGroup::U));
-  const uint16_t* __restrict__ sw = reinterpret_cast<const uint16_t*>(pick(a.grp, g, &LrFwdGroup::sw));
-  uint16_t* __restrict__ y = reinterpret_cast<uint16_t*>(pick(a.grp, g, &LrFwdGroup::y));
+  const auto* gp = kernel_args<LrArgs>()->grp + g;  // the group's pointers: scalar loads at a uniform offset
+  const uint16_t* __restrict__ x = reinterpret_cast<const uint16_t*>(gp->x);
+  const uint16_t* __restrict__ z = reinterpret_cast<const uint16_t*>(gp->z);
+  const uint16_t* __restrict__ U = reinterpret_cast<const uint16_t*>(gp->U);
+  const uint16_t* __restrict__ sw = reinterpret_cast<const uint16_t*>(gp->sw);
+  uint16_t* __restrict__ y = reinterpret_cast<uint16_t*>(gp->y);
   const int chunk = lb % a.nch, sgp = lb / a.nch;  // NWV wavefronts: one chunk, NWV consecutive runs
   const int D = a.D, Tn = a.Tn, R = a.R, RK = a.RK;
   const int dl = chunk * 128 + 8 * n;  // first channel of the lane's octet
@@ -166,7 +177,7 @@ void lr_fwd_mfma(LrArgs a) {
   const rsrc_t rz = run_rsrc(z + rrow * zld, Tn - rb, zld * 2);
   const int zrp = ZE ? a.zrp : 0;
   const bool zrow_mine = ZE && n % a.nch == chunk;  // this wavefront writes row n of each tile's z_eff
-  const rsrc_t rze = ZE ? run_rsrc((const uint16_t*)pick(a.grp, g, &LrFwdGroup::zeff) + rrow * zrp, Tn - rb, zrp * 2)
+  const rsrc_t rze = ZE ? run_rsrc((const uint16_t*)gp->zeff + rrow * zrp, Tn - rb, zrp * 2)
                         : make_rsrc(z, 0);
   // y: the lane's row-4q octet (head yh, relative to head yh0's row rb)
   const int lane_off = chv ? (((yh - yh0) * Tn + 4 * q) * yhd + dl - yh * yhd) * 2 : kOobLane;

@@ -10,11 +10,19 @@ namespace {
 
 // Wavefronts per problem: runs of about 8 tiles, at most 4096 wavefronts
 // (4 per SIMD).  B4 T4096 D2048: 2048 wavefronts (31.4 us, 31.9 at 4096);
-// B2 T8192 D4096: 4096 (61.8 us, 64.0 at 2048).
+// B2 T8192 D4096: 4096 (61.8 us, 64.0 at 2048).  Problems below 8 tiles for
+// each of kFwdFillWaves wavefronts take shorter runs instead of fewer
+// wavefronts: a run's tiles are a serial chain of 1-2 us each, which nothing
+// else on an idle chip hides.  Forward, runs of 8 tiles -> filled (bf16, with
+// static): B2 T512 D256 R15 14.5 -> 5.5 us, B3 T1537 D1000 R7 W3 17.1 -> 9.6,
+// B2 T2048 D2048 R16 19.4 -> 10.1, B4 T2048 D2048 R31 28.9 -> 21.7; filling
+// 1024 only: 5.5, 10.0, 12.4, 28.2 us.
+constexpr int kFwdFillWaves = 2048;
 inline int fwd_target_waves(const LrProblem& p) {
   const int64_t tiles = p.B * ((p.T + 15) / 16) * ((p.D + 127) / 128);
   const int64_t w = tiles / 8;
-  return (int)(w < 1 ? 1 : w > 4096 ? 4096 : w);
+  if (w < kFwdFillWaves) return (int)(tiles < kFwdFillWaves ? tiles : kFwdFillWaves);
+  return (int)(w > 4096 ? 4096 : w);
 }
 
 // One rank chunk without the z_eff writer: at most two wavefronts per SIMD, on
