@@ -462,6 +462,34 @@ int64_t lr_bwd_max_run_tiles(const LrProblem& p) {
 
 namespace {
 
+// Tiles per run of lr_bwd_t32: a CU holds one of its workgroups, so a launch
+// takes ceil(workgroups / 256) rounds of a run's length each, and a few
+// workgroups past a round cost as much as a full one (B1 T8192 D768 R15 + static
+// W 8: runs of 3 tiles are 258 workgroups and took 48 us, runs of 4 31 us; B3
+// T4788 D3712 R32: 270 workgroups 163 us, 225 116 us).  Of the run
+// lengths that fill one to eight rounds, the one with the least time by a
+// model: per round a launch's start and end (6 us) and the run's tiles, and
+// every run's dU partial written and read once.  dflt: no such length (more
+// sequences than eight rounds hold).
+int64_t t32_run_tiles(const LrProblem& p, int64_t ntile, int64_t cols, int64_t dflt) {
+  constexpr int64_t kCus = 256;
+  const double tile_us = 0.6 * (p.W < 2 ? 2 : p.W > 8 ? 8 : p.W) * (bwd_rc(p) == 2 ? 1.25 : 1.0);
+  const double part_us = (double)(p.R + (p.static_w ? 1 : 0)) * p.W * p.D * 8 / 5e6;
+  int64_t best = dflt;
+  double best_us = -1;
+  for (int64_t rounds = 1; rounds <= 8; ++rounds) {
+    const int64_t per_seq = rounds * kCus / (p.B * cols);  // runs a sequence may take
+    if (per_seq < 1) continue;
+    const int64_t seg = (ntile + per_seq - 1) / per_seq, runs = p.B * ((ntile + seg - 1) / seg);
+    const double us = rounds * (6.0 + seg * tile_us) + runs * part_us;
+    if (best_us < 0 || us < best_us) {
+      best = seg;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 // split: the passes of ranks form dz and dU in one launch (bwd_dx_split); each
 // run is then nrp workgroup rows, so runs are nrp times as long for the same
 // number of workgroups (and the dU partials nrp times fewer).
@@ -479,10 +507,11 @@ LrBwdArgs make_bwd_args(const LrProblem& p, int target_waves, bool split) {
   a.ncg = (a.nch + ncw - 1) / ncw;
   const int64_t ntile = (p.T + rows - 1) / rows;
   a.nrp = split ? bwd_rank_passes(p) : 1;
+  const int64_t cap = lr_bwd_max_run_tiles(p) * 16 / rows;  // >= 1 (lr_mfma_ok)
   int64_t seg = (p.B * ntile * a.ncg * ncw * a.nrp + target_waves - 1) / target_waves;
+  if (t32) seg = t32_run_tiles(p, ntile, (int64_t)a.ncg * a.nrp, seg);
   if (seg < 1) seg = 1;
   if (seg > ntile) seg = ntile;
-  const int64_t cap = lr_bwd_max_run_tiles(p) * 16 / rows;  // >= 1 (lr_mfma_ok)
   if (seg > cap) seg = cap;
   a.seg = (int)seg;
   a.nspb = (int)((ntile + seg - 1) / seg);
