@@ -74,6 +74,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   static_assert((RC == 1 && W <= 8) || (RC == 2 && W <= 4), "operands and accumulators of one pass");
   constexpr int NW = 8;                     // wavefronts: 256 channels
   constexpr int NR = W + 7;                 // x rows 8q-W+1 .. 8q+7 per lane
+  // halo rows of x from the neighbour lanes where the registers hold the previous
+  // tile's (B4 T4096 D2048 backward R16 59.2 -> 58.5 us, R63 + static 151.5 -> 148.9;
+  // two rank chunks with dx spill with it: 123 -> 129 us), else loaded
+  constexpr bool HX = W > 1 && ((RC == 1 && W <= 4) || DXM == 3);
+  constexpr int NX = HX ? 8 : NR;           // x rows loaded per lane
   constexpr int NO = W > 1 ? W - 1 : 1;     // open rows of a group (none at W 1)
   constexpr int kFirstOpen = 9 - W;         // rows kFirstOpen .. 7 take the group below's sums
   constexpr bool NODX = DXM == 3;
@@ -154,7 +159,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // read 0; a tile past the run the out-of-range offset kOobTile).  dy and z of
   // the tile after the run are read too: its first rows close the run's last dx rows.
   struct TileIn {
-    uint32_t xr[NR], dyr[8];
+    uint32_t xr[NX], dyr[8];
     ZR zraw[RC == 2 ? 1 : 2];
     u32x4 z32[RC == 2 ? 2 : 1];
   };
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const bool ylive = NODX ? tile < tile1 : tile <= tile1;
     const int toff = ylive ? (tile * 32 - rb) * rowb : kOobTile;
 #pragma unroll
-    for (int m = 0; m < NR; ++m) in.xr[m] = LV::load(rx, xlane_off + xtoff + (m - (W - 1)) * xrowb);
+    for (int m = 0; m < NX; ++m) in.xr[m] = LV::load(rx, xlane_off + xtoff + (m + 8 - NX) * xrowb);
 #pragma unroll
     for (int m = 0; m < 8; ++m) in.dyr[m] = LV::load(rdy, lane_off + toff + m * rowb);
 #pragma unroll
@@ -178,6 +183,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
 #pragma unroll
   for (int i = 0; i < NBUF; ++i) load_tile(in[i], tile0 + i);
+  // HX: x rows 8q-W+1 .. 8q-1 are own rows of the lane group above (lane - 16),
+  // or for group 0 those of group 3 in the tile before (prev: loaded for the run's
+  // first tile), passed with one ds_bpermute each.
+  uint32_t prev[NO];
+  if constexpr (HX) {
+#pragma unroll
+    for (int m = 0; m < W - 1; ++m)
+      prev[m] = LV::load(rx, (chv ? col * 2 : kOobLane) + (tile0 * 32 - kofs + m - (W - 1) - rb) * xrowb);
+  }
   __builtin_amdgcn_sched_barrier(0);  // the first tile's loads go out before the U staging waits
 
   // ---- U_eff operands of the wavefront's 32 channels (rows >= R of U and
@@ -390,10 +404,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   auto do_tile = [&](int it, TileIn& in) {
     const int tile = tile0 + it;
     float xf[NR][2], dyf[8][2];
+    const int above = ((lane + 48) & 63) << 2;  // ds_bpermute byte index of lane - 16
 #pragma unroll
-    for (int m = 0; m < NR; ++m)
+    for (int m = 0; m < NR; ++m) {
+      uint32_t v;
+      if (HX && m < W - 1) {
+        const uint32_t own = in.xr[HX ? (m + 9 - W) % NX : 0];  // row 8q+9-W+m
+        v = (uint32_t)__builtin_amdgcn_ds_bpermute(above, (int)(q == 3 ? prev[m % NO] : own));
+        prev[m % NO] = own;
+      } else {
+        v = in.xr[m - (NR - NX)];
+      }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) xf[m][j] = Mma16<T>::to_f(LV::elem(in.xr[m], j));
+      for (int j = 0; j < 2; ++j) xf[m][j] = Mma16<T>::to_f(LV::elem(v, j));
+    }
 #pragma unroll
     for (int m = 0; m < 8; ++m)
 #pragma unroll
