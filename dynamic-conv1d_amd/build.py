@@ -3,8 +3,8 @@
     python dynamic-conv1d_amd/build.py [--jobs N] [--host-sanitize]
 
 Each csrc/*.hip translation unit is compiled in parallel to _build/*.o and
-linked into dynconv/libdynconv.so.  Always rebuilds (the driver's "does it
-build" check calls this on every round).
+linked into dynconv/libdynconv.so; csrc/torch_binding.cpp (host code only) is
+compiled against the installed torch into dynconv/_binding.so.  Always rebuilds.
 
 --host-sanitize builds dynconv/libdynconv_hostsan.so instead (objects in
 _build_hostsan/): the host code (argument checks, launch plans, the range
@@ -31,6 +31,8 @@ OUT_SAN = os.path.join(HERE, "dynconv", "libdynconv_hostsan.so")
 HOST_SAN = ["-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fsanitize=undefined",
             "-Xarch_host", "-fno-sanitize-recover=undefined", "-Xarch_host", "-fno-omit-frame-pointer"]
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
+BINDING_SRC = os.path.join(CSRC, "torch_binding.cpp")
+BINDING_OUT = os.path.join(HERE, "dynconv", "_binding.so")
 
 ARCH = "gfx950"
 # -packed-fp32-ops: keep hipcc from emitting packed fp32 VALU ops (v_pk_*_f32).
@@ -73,6 +75,32 @@ def _compile(src: str, extra: list, bdir: str = BUILD) -> tuple:
     return src, obj, r.returncode, err, time.time() - t0
 
 
+def build_binding(verbose: bool = True) -> str:
+    """Compile csrc/torch_binding.cpp (host code) into dynconv/_binding.so with g++."""
+    import sysconfig
+
+    import torch
+
+    t = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    tmp = BINDING_OUT + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-deprecated",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DTORCH_VERSION_BUILT="{torch.__version__}"',
+           "-I", INCLUDE, "-isystem", os.path.join(t, "include"),
+           "-isystem", os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
+           BINDING_SRC, "-o", tmp, "-L", os.path.join(t, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    t0 = time.time()
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if verbose or r.returncode:
+        print(f"[build] torch_binding.cpp: {'ok' if r.returncode == 0 else 'FAILED'} ({time.time() - t0:.1f}s)", flush=True)
+    if r.returncode:
+        raise RuntimeError(f"compiling torch_binding.cpp failed:\n{r.stderr[-4000:]}")
+    os.replace(tmp, BINDING_OUT)
+    return BINDING_OUT
+
+
 def build(jobs: int = 0, extra=None, verbose: bool = True, host_sanitize: bool = False) -> str:
     extra = list(extra or []) + (HOST_SAN if host_sanitize else [])
     bdir, out = (BUILD_SAN, OUT_SAN) if host_sanitize else (BUILD, OUT)
@@ -82,6 +110,7 @@ def build(jobs: int = 0, extra=None, verbose: bool = True, host_sanitize: bool =
     objs = []
     failed = []
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        binding = None if host_sanitize else ex.submit(build_binding, verbose)
         for src, obj, rc, err, dt in ex.map(lambda s: _compile(s, extra, bdir), srcs):
             if verbose:
                 print(f"[build] {os.path.basename(src)}: {'ok' if rc == 0 else 'FAILED'} ({dt:.1f}s)", flush=True)
@@ -92,6 +121,8 @@ def build(jobs: int = 0, extra=None, verbose: bool = True, host_sanitize: bool =
             objs.append(obj)
     if failed:
         raise RuntimeError(f"hipcc failed for: {', '.join(os.path.basename(f) for f in failed)}")
+    if binding is not None:
+        binding.result()
     tmp = out + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)

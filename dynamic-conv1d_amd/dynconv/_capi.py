@@ -53,11 +53,27 @@ SIGNATURES = {
 
 _lib = None
 _lock = threading.Lock()
+# The native autograd binding (csrc/torch_binding.cpp, built beside the library),
+# once load() has given it the library; None before that, or where it was not
+# built for this torch: the Functions in headwise.py, lowrank.py and modules.py
+# take every call then, as they take each call that the binding declines.
+binding = None
+
+
+def _load_binding(path: str):
+    try:
+        from . import _binding as b
+    except ImportError:
+        return None
+    if b.torch_version != torch.__version__:
+        return None
+    b.init(path)
+    return b
 
 
 def load(path: str = LIB_PATH):
     """Load (once) and return the ctypes handle of libdynconv.so."""
-    global _lib
+    global _lib, binding
     if _lib is not None:
         return _lib
     with _lock:
@@ -76,6 +92,7 @@ def load(path: str = LIB_PATH):
         ver = lib.dc_abi_version()
         if ver != ABI_VERSION:
             raise RuntimeError(f"libdynconv.so ABI version {ver}, expected {ABI_VERSION}")
+        binding = _load_binding(path)
         _lib = lib
     return _lib
 

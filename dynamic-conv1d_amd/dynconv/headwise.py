@@ -11,7 +11,7 @@ from . import _capi
 
 
 class _HeadwiseDynamicConvolutionFn(torch.autograd.Function):
-    """Autograd glue; mirrors headwise.py:218-309."""
+    """Autograd glue; mirrors headwise.py:218-309.  Plain calls take its native form (_capi.binding)."""
 
     @staticmethod
     @_capi.on_tensor_device
@@ -89,6 +89,10 @@ def headwise_dynamic_convolution(
     float32) and round y and each gradient once to its tensor's dtype, as the
     reference stores its fp32 results; one dtype throughout takes no copies.
     """
+    if _capi.binding is not None:
+        y = _capi.binding.headwise(x, weight, static_w, residual)
+        if y is not None:
+            return y
     assert x.is_cuda and x.is_contiguous()
     if static_w is not None:
         assert static_w.is_cuda and static_w.is_contiguous()

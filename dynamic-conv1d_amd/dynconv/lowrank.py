@@ -25,7 +25,7 @@ def _zeff_buffers(lib, n, B, T, D, R, W, dtype, has_static, device):
 
 
 class _LowrankDynamicConvolutionFn(torch.autograd.Function):
-    """Autograd glue; mirrors lowrank.py:214-299."""
+    """Autograd glue; mirrors lowrank.py:214-299.  Plain calls take its native form (_capi.binding)."""
 
     @staticmethod
     @_capi.on_tensor_device
@@ -108,6 +108,10 @@ def lowrank_dynamic_convolution(
     Preconditions as lowrank.py:328-337, plus (checked here, assumed by the
     reference) one shared dtype for x, z and U and W*D columns in U.
     """
+    if _capi.binding is not None:
+        y = _capi.binding.lowrank(x, z, U, static_w, residual)
+        if y is not None:
+            return y
     assert x.is_cuda and x.is_contiguous()
     assert z.is_cuda and z.is_contiguous()
     assert U.is_cuda and U.is_contiguous()

@@ -162,6 +162,14 @@ class GroupedLowRankDynamicShortConvolution(nn.Module):
 
     def forward(self, x: torch.Tensor, pre_z: torch.Tensor):
         G, R = self.groups, self.R
+        # proj_in and the grouped operator as one native node, on the same conditions as
+        # _module_proj_in: nothing else may be looking at the projection
+        if (_capi.binding is not None and _plain_linear(self.proj_in)
+                and not torch.is_autocast_enabled(pre_z.device.type)):
+            ys = _capi.binding.grouped_module(x, pre_z, self.proj_in.weight, self.proj_out, self.proj_out_bias,
+                                              self.head_dim)
+            if ys is not None:
+                return ys
         zs = list(_module_proj_in(self.proj_in, pre_z, G, R))  # one GEMM for every group
         Us = [self.proj_out[g] for g in range(G)]
         sws = [self.proj_out_bias[g] for g in range(G)]
