@@ -232,7 +232,10 @@ struct ZRaw {
 // dx of the backward over all kernel ranks in one launch (lowrank_mfma_dx.hip;
 // the passes of ranks then form dz and dU only).
 template <typename T>
-hipError_t lr_dx_mfma_launch(const LrProblem* p, int G);
+hipError_t lr_dx_mfma_launch(const LrProblem* p, int G, const void* const* z, int zld);
+// Its shapes: the packed U operands of all taps and ranks in one workgroup's LDS
+// (W x 32-rank chunks x 8 KiB, at most 128 KiB), the look-ahead in one lane group.
+inline bool lr_dx_split_shape(int64_t RK, int64_t W) { return W <= 8 && RK <= 128 && W * ((RK + 31) / 32) <= 16; }
 
 inline bool aligned_to(const void* p, int a) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 

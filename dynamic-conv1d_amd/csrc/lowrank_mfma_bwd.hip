@@ -396,12 +396,14 @@ inline int bwd_rank_passes(const LrProblem& p) {
 // R73 + static W2, 3 passes, against 0.02 + 2%).
 constexpr int kBwdMaxBf16DxPasses = 4;
 constexpr int kBwdMaxBf16DxRankPasses = 2;
-// Passes of ranks at W <= 4 up to kernel rank 128 with dy in [B, T, D]: the
-// passes form dz and dU only (DXM 3) and lr_dx_mfma forms dx over all ranks in
-// one launch, rounded once (no fp32 accumulator).
+// Passes of ranks with dy in [B, T, D] whose dx fits one launch
+// (lr_dx_split_shape: W <= 8 up to kernel rank 64, W 5 / 4 up to 96 / 128): the
+// passes form dz and dU only (DXM 3) and lr_dx_t32 forms dx over all ranks and
+// taps in one launch, rounded once (no fp32 accumulator).  Passes of taps alone
+// (two rank chunks above W 4) keep dx: split off it measured 160 -> 166 us at B4
+// T4096 D2048 R31 + static W 8.
 inline bool bwd_dx_split(const LrProblem& p) {
-  const int64_t rk = p.R + (p.static_w ? 1 : 0);
-  return bwd_rank_split(p) && p.W <= 4 && rk <= 128 && p.yhd() == p.D;
+  return bwd_rank_split(p) && lr_dx_split_shape(p.R + (p.static_w ? 1 : 0), p.W) && p.yhd() == p.D;
 }
 // The workspace keeps room for the accumulator whether or not dx is split off:
 // the size queries do not see dy's layout, on which the split depends.
@@ -761,14 +763,22 @@ hipError_t launch_bwd(const LrProblem* p, int G) {
       audit_bwd_pass(b, f.W, f32);
       continue;
     }
-    if (dxs) {  // all passes of ranks in one launch, from the whole problem's arguments
-      if (i > 0) continue;
-      b = a;
+    if (dxs) {  // all passes of ranks of these taps in one launch, from the whole problem's ranks
+      if (f.rofs > 0) continue;
+      b.R = a.R;
+      b.RK = a.RK;
+      b.accdx = 0;
       b.residual = 0;
+      for (int g = 0; g < G; ++g)
+        b.grp[g].sw = p[g].static_w ? (const void*)((const T*)p[g].static_w + f.kofs * D) : nullptr;
     }
     if ((e = dispatch_bwd_kernel<T>(b, f.W, rc, f32, p[0].stream)) != hipSuccess) return e;
   }
-  if (dxs && (e = lr_dx_mfma_launch<T>(p, G)) != hipSuccess) return e;
+  if (dxs) {
+    const void* zs[kMaxGroups];
+    for (int g = 0; g < G; ++g) zs[g] = a.grp[g].z;
+    if ((e = lr_dx_mfma_launch<T>(p, G, zs, a.zld)) != hipSuccess) return e;
+  }
   // The last pass stores dx rows 0 .. T-1-kofs of its taps kofs ..; the rows
   // after those (no terms of its taps) are rounded from the accumulator here
   // (passes that split only the ranks have kofs 0: nothing left).

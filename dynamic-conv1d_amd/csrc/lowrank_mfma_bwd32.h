@@ -134,7 +134,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     part_dz += rofs;
     part_du += (int64_t)rofs * a.uld;
   }
-  const int kofs = ACC ? a.kofs : 0;  // a later pass of taps: x read, dx stored kofs rows earlier
+  const int kofs = ACC || NODX ? a.kofs : 0;  // a later pass of taps: x read, dx stored kofs rows earlier
   const float res = a.residual && a.kofs == 0 ? 1.f : 0.f;
   // head-major dy: the wavefront's channels lie in one head (yhd % 64 == 0), whose [T, yhd] block rdy covers
   const int yhd = a.yhd, head = d0 / yhd;

@@ -3,7 +3,7 @@
 // lowrank_mfma_fwd_wide.hip (9 <= W <= 16, and the last 16 taps above W 16).
 #pragma once
 
-#include "lowrank_mfma_fwd_kernel.h"
+#include "lowrank_mfma_t32.h"
 
 namespace dc {
 namespace {
@@ -89,6 +89,26 @@ hipError_t launch_fwd(const LrProblem* p, int G) {
     }
     audit_range(run_rsrc_bytes((int64_t)heads * a.Tn + a.Tn, (int64_t)a.yhd * 2), kOobTile - 15 * (int64_t)a.yhd * 2);
     return hipSuccess;
+  }
+  if constexpr (!ACC && W <= 8 && (RC == 2 || RC == 4)) {
+    // 32 ranks to a product (lr_fwd_t32): z rows of whole 16-byte octets, or of R % 8
+    // == 7 ranks (R + 1 a power of two: a module's ranks with a static filter); other
+    // ranks keep the 16-rank kernels.  The z_eff rows are stored in octets.
+    bool zal = a.R % 8 == 0 && a.zld % 8 == 0;
+    for (int g = 0; g < G; ++g) zal = zal && aligned_to(p[g].z, 16);
+    const int64_t cap = lr_fwd_max_run_tiles(p[0]) / 2, ntile = (p[0].T + 31) / 32;
+    if ((zal || a.R % 8 == 7) && a.zrp % 8 == 0 && cap >= 1) {
+      const int nwv = t32_wg_waves(W, RC / 2);
+      int64_t seg = t32_run_tiles(p[0].B * ntile * a.nch);
+      seg = seg > cap ? cap : seg;
+      a.zvec = zal;
+      a.seg = (int)(seg > ntile ? ntile : seg);
+      a.nspb = (int)((ntile + a.seg - 1) / a.seg);
+      a.nseg = (int)(p[0].B * a.nspb);
+      a.nblk1 = ((a.nseg + nwv - 1) / nwv) * a.nch;
+      a.nblk = G * a.nblk1;
+      return lr_fwd_t32_launch<T>(a, W, RC / 2, p[0].stream);
+    }
   }
   if constexpr (ACC) {  // a later pass of taps (no z_eff writer)
     if (a.zvec)

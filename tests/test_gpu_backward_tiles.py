@@ -25,7 +25,11 @@ CASES = (
     # ranks around the chunks
     + [(2, 45, 64, R, 2, st, bf16) for R, st in ((1, False), (3, True), (15, True), (17, False), (32, False))]
     # passes of 32 ranks in one launch (dx in a launch of its own): the static rank in, and alone in, the last
-    + [(2, 100, 72, R, W, st, bf16) for R, W, st in ((40, 3, True), (63, 4, True), (64, 4, True), (127, 2, True))]
+    + [(2, 100, 72, R, W, st, bf16) for R, W, st in ((40, 3, True), (63, 4, True), (64, 4, True), (127, 2, True),
+                                                        (63, 5, True), (40, 6, False), (63, 8, True), (80, 5, True),
+                                                        (64, 8, False), (127, 4, True), (96, 1, False))]
+    # its runs of tiles: the dx launch's carry over tiles, the tile after a run
+    + [(1, 70100, 136, 63, 4, True, bf16), (1, 70100, 136, 40, 8, True, fp16)]
     # passes of taps (dx of the earlier passes added) at one and two rank chunks, rows 32 apart from the halo
     + [(1, 97, 64, 16, 12, False, bf16), (1, 97, 64, 31, 7, True, fp16), (1, 33, 64, 20, 20, True, bf16)]
     # several runs to a sequence: the tile after a run closes its last rows

@@ -13,7 +13,10 @@ from dynconv import lowrank as lr_mod
 pytestmark = pytest.mark.gpu
 
 # T x D in tiles of 16 x 128: 2048 wavefronts take one tile each up to 2048 tiles, then 2, .. 8
-CASES = [(1, T, 264, R, st, W) for T in (10900, 11000, 40001) for R, st, W in ((15, True, 3), (31, True, 4), (16, False, 8),
+# ranks of 32 to a product: whole octets, octets and a static rank, R % 8 == 7; other ranks beside them
+RANKS = [(24, True), (32, False), (23, True), (31, False), (63, True), (56, True), (64, False), (17, True), (50, False)]
+CASES = [(2, T, 136, R, st, W) for T, W in ((1, 4), (31, 1), (33, 8), (70, 5)) for R, st in RANKS]
+CASES += [(1, T, 264, R, st, W) for T in (10900, 11000, 40001) for R, st, W in ((15, True, 3), (31, True, 4), (16, False, 8),
                                                                              (40, False, 5), (15, True, 12))]
 
 
