@@ -20,14 +20,19 @@
 // pre_z straight into MFMA operands (v_mfma_f32_16x16x32: lane 16q + n holds
 // row n, K elements 8q .. 8q+7 of each 32-wide step).
 //
-// Backward (proj_bwd): one pass over pre_z.  A workgroup owns 256 channels
-// (4 wavefronts of 64) of one run of 16-row tiles; lane 16q + n holds rows
-// 4q .. 4q+3, channels 4n .. 4n+3 of its wavefront's 64.  Per tile the
-// workgroup stages the 16 rows of dz in LDS twice, row-major (the A operand
-// of dpre_z = dz W_in, K = 32 ranks) and rank-major (dz^T, the A operand of
-// dW_in += dz^T pre_z, K = 16 rows).  The W_in operands of the wavefront's 64
-// channels sit in registers for the whole run.  dW_in is written as one fp32
+// Backward (proj_bwd): one pass over pre_z.  A workgroup owns 256 channels (8
+// wavefronts of 32) of one run of 32-row tiles; lane 16q + n holds rows 8q ..
+// 8q+7, channels 2n, 2n+1 of its wavefront's 32.  The tile's dz rows are staged
+// once in LDS: row-major reads are the A operand of dpre_z = dz W_in (K = 32
+// ranks), transposing reads that of dW_in += dz^T pre_z (K = the 32 rows).  The
+// W_in operands sit in registers for the whole run.  dW_in is written as one fp32
 // partial per run and summed by reduce_partials (fixed order: deterministic).
+// Against 16-row tiles of 4 wavefronts (K = 16 rows to a product, dz staged twice
+// with a division per element and tile, 32 runs for every shape), bf16: M 8192 K
+// 2048 G3 R31 45 -> 28.6 us, M 2756 K 1792 28.6 -> 19.8, M 16384 K 4096 107 -> 103
+// (then bound by the tile's latency at two wavefronts per SIMD; a third and fourth
+// tile in flight: 108).  Stores are nontemporal (default stores: 31 -> 51 us at M
+// 16384 K 2048 G1 R31), loads are not (35 against 29 us at M 8192 K 2048).
 #include "lowrank_mfma.h"
 
 namespace dc {
@@ -184,173 +189,193 @@ __global__ __launch_bounds__(256 * KS) void proj_fwd(ProjArgs a) {
 }
 
 // --------------------------------------------------------------- backward
-template <typename T, int NB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB <= 6 ? 2 : 1, 8))) void proj_bwd(ProjArgs a) {
+template <typename T, int NB, int NG>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) void proj_bwd(ProjArgs a) {
   constexpr int NP = NB * 16;          // ranks padded to whole 16-rank chunks (zero past N)
   constexpr int N32 = (NP + 31) / 32;  // 32-rank steps of the dpre_z product
-  constexpr int NP32 = N32 * 32;       // ranks of the row-major dz tile (zero past N)
-  constexpr int DROW = NP32 * 2 + 16;  // bytes per row of the row-major dz tile (16-byte pad)
-  constexpr int TROW = 16 * 2 + 8;     // bytes per rank of the rank-major tile (8-byte pad)
-  __shared__ __attribute__((aligned(16))) uint8_t dzr[2][16 * DROW];  // [row][rank]
-  __shared__ __attribute__((aligned(16))) uint8_t dzt[2][NP * TROW];  // [rank][row]
+  constexpr int NP32 = N32 * 32;       // ranks of a staged dz row (zero past N)
+  constexpr int DROW = NP32 * 2 + 16;  // bytes per staged row (16-byte pad)
+  constexpr int TILE = 32 * DROW;
+  constexpr int NBUF = 2;              // tiles of pre_z in flight (dz: two)
+  __shared__ __attribute__((aligned(16))) uint8_t dzl[2][TILE];  // [row][rank], alternating
 
-  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int lane = threadIdx.x & 63, wave = wave_id(), tid = (int)threadIdx.x;
   const int q = lane >> 4, n = lane & 15;
   const int blk = xcd_remap(blockIdx.x, a.nblk);
   const int cg = blk % a.ncg, run = blk / a.ncg;
   const int M = a.M, K = a.K, N = a.N, R = a.R;
-  const int d0 = cg * 256 + wave * 64;   // the wavefront's first channel
-  const int col = d0 + 4 * n;            // the lane's first channel (K % 8 == 0: 4 channels wholly in or out)
+  const int col = cg * 256 + wave * 32 + 2 * n;  // the lane's first channel (K % 8 == 0: both in or out)
   const bool chv = col < K;
-  const int ntile = (M + 15) >> 4;
+  const int ntile = (M + 31) >> 5;
   const int tile0 = run * a.seg, tile1 = min(tile0 + a.seg, ntile);
-  const int r0 = tile0 * 16;
-  const int nrow = max(min(M - r0, (tile1 - tile0) * 16), 0);
+  const int r0 = tile0 * 32;
+  const int nrow = max(min(M - r0, (tile1 - tile0) * 32), 0);
   const rsrc_t rp = make_rsrc_wave<kProjOob>(a.pre + (int64_t)min(r0, M) * K, (int64_t)nrow * K * 2);
   const rsrc_t rd = make_rsrc_wave<kProjOob>(a.dpre + (int64_t)min(r0, M) * K, (int64_t)nrow * K * 2);
-  // the lane's row-4q channels in pre_z / dpre_z; lanes past K (chv false)
+  // the lane's row-8q channels in pre_z / dpre_z; lanes past K (chv false)
   // take kProjOob alone, never kProjOob plus a row offset (that sum would
   // overflow int32 and wrap back into the range)
-  const int lane_off = (4 * q * K + col) * 2;
+  const int lane_off = (8 * q * K + col) * 2;
 
+  // dz staging: group g's 32 rows of a tile are 32 R contiguous elements; thread
+  // tid takes elements 2 tid, 2 tid + 1 (+ 1024 j) of each group, whose rows and
+  // ranks in the tile, and so their LDS places, are the same for every tile.
+  constexpr int NJ = (NP / NG * 16 + 511) / 512;  // pairs per thread and group: 16 R pairs, R = N / NG
+  int place[NJ][2];                          // byte in a staged tile (group 0; + 2 R per group), or -1
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int el = 2 * (tid + 512 * j) + e, row = el / R;
+      place[j][e] = row < 32 ? row * DROW + (el - row * R) * 2 : -1;
+    }
+  // two tiles ahead like pre_z: loads retire in order, so a wait for dz loads issued
+  // after a tile's pre_z loads would wait for those too (3.3 us a tile)
+  uint32_t sv[2][NG][NJ][2];
+  auto load_dz = [&](int tile, uint32_t(&sv)[NG][NJ][2]) {
+    const int nel = max(min(M - tile * 32, 32), 0) * R;  // elements of the tile (0 past the run)
+    const bool live = tile < tile1;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const uint16_t* base = a.dz[g] + (int64_t)tile * 32 * R;
+      const rsrc_t rz = make_rsrc_wave<kProjOob>(base, live ? (int64_t)nel * 2 : 0);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int el = 2 * (tid + 512 * j);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) sv[g][j][e] = bload16(rz, (el + e) * 2);
+      }
+    }
+  };
+  auto store_dz = [&](int b, const uint32_t(&sv)[NG][NJ][2]) {
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          if (place[j][e] >= 0)
+            *reinterpret_cast<uint16_t*>(&dzl[b][place[j][e] + 2 * R * g]) = (uint16_t)sv[g][j][e];
+      }
+    }
+  };
+  // pre_z rows 8q .. 8q+7 of a tile, the lane's 2 channels (rows past the run read 0)
+  auto load_pre = [&](int tile, uint32_t(&pr)[8]) {
+    const bool live = chv && tile < tile1;
+    const int toff = (tile - tile0) * 32 * K * 2;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) pr[i] = bload32(rp, live ? lane_off + toff + i * K * 2 : kProjOob);
+  };
+
+  uint32_t pre[NBUF][8];
+#pragma unroll
+  for (int b = 0; b < NBUF; ++b) {
+    if (b < 2) load_dz(tile0 + b, sv[b & 1]);
+    load_pre(tile0 + b, pre[b]);
+  }
+  // ranks N .. NP32-1 of both staged tiles stay zero
+  for (int e = tid; e < 2 * 32 * (NP32 - N); e += 512) {
+    const int b = e / (32 * (NP32 - N)), rem = e - b * 32 * (NP32 - N), row = rem / (NP32 - N);
+    *reinterpret_cast<uint16_t*>(&dzl[b][row * DROW + (N + rem - row * (NP32 - N)) * 2]) = 0;
+  }
   // W_in operands of the dpre_z product (B of v_mfma_f32_16x16x32, K = ranks):
   // step s, channel j: ranks 32s + 8q .. +7 of channel col + j, packed.
-  u32x4 wop[N32][4];
+  u32x4 wop[N32][2];
   {
     const rsrc_t rw = make_rsrc_wave<kProjOob>(a.w, (int64_t)N * K * 2);
 #pragma unroll
     for (int s = 0; s < N32; ++s) {
-      u32x2 rows8[8];
+      uint32_t rows8[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const int c = 32 * s + 8 * q + e;
-        rows8[e] = bload64(rw, chv && c < N ? (c * K + col) * 2 : kProjOob);
+        rows8[e] = bload32(rw, chv && c < N ? (c * K + col) * 2 : kProjOob);
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int h = 0; h < 4; ++h)
-          wop[s][j][h] = elem16x2(rows8[2 * h], j) | (elem16x2(rows8[2 * h + 1], j) << 16);
+          wop[s][j][h] = __builtin_amdgcn_perm(rows8[2 * h + 1], rows8[2 * h], j ? 0x07060302u : 0x05040100u);
     }
   }
-
-  f32x4 dw[NB][4];
+  f32x4 dw[NB][2];
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) dw[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // dz tile staging: NP32 x 16 elements, ~NP32 / 16 per thread; rank c is group
-  // c / R, rank c % R (G separate tensors), zero past N and past M.
-  constexpr int SPT = (NP32 * 16 + 255) / 256;
-  uint32_t sv[SPT];
-  auto load_dz = [&](int tile) {
-#pragma unroll
-    for (int i = 0; i < SPT; ++i) {
-      const int e = i * 256 + (int)threadIdx.x;
-      const int row = e / NP32, c = e - row * NP32;
-      const int m = tile * 16 + row;
-      // an unconditional load from a valid address (group 0's first element when
-      // the element lies outside the tile), so no load sits under a branch
-      const bool ok = e < NP32 * 16 && c < N && m < M && tile < tile1;
-      const int g = ok ? c / R : 0;
-      const uint16_t* src = ok ? pick4(a.dz, g) + ((int64_t)m * R + (c - g * R)) : a.dz[0];
-      const uint32_t v = *src;
-      sv[i] = ok ? v : 0u;
-    }
-  };
-  auto store_dz = [&](int b) {
-#pragma unroll
-    for (int i = 0; i < SPT; ++i) {
-      const int e = i * 256 + (int)threadIdx.x;
-      if (e >= NP32 * 16) break;
-      const int row = e / NP32, c = e - row * NP32;
-      *reinterpret_cast<uint16_t*>(&dzr[b][row * DROW + c * 2]) = (uint16_t)sv[i];
-      if (c < NP) *reinterpret_cast<uint16_t*>(&dzt[b][c * TROW + row * 2]) = (uint16_t)sv[i];
-    }
-  };
-  // pre_z rows 4q .. 4q+3 of a tile, the lane's 4 channels (rows past the run read 0)
-  auto load_pre = [&](int tile, u32x2(&pr)[4]) {
-    const bool live = chv && tile < tile1;
-    const int toff = (tile - tile0) * 16 * K * 2;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) pr[i] = bload64<kNt>(rp, live ? lane_off + toff + i * K * 2 : kProjOob);
-  };
-
-  u32x2 pa[4], pb[4];
-  load_dz(tile0);
-  store_dz(0);
-  load_pre(tile0, pa);
+    for (int j = 0; j < 2; ++j) dw[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  store_dz(0, sv[0]);
   __syncthreads();
-  auto compute = [&](int tile, int b, const u32x2(&pr)[4]) {
-    // dpre_z = dz W_in: A = dz row n, ranks 32s + 8q .. +7
-    f32x4 acc[4];
+
+  // Transposing reads of dz^T: lane a + 4i of group q addresses row 8q + i (+ 4),
+  // ranks 4a ..; it receives rank n of rows 8q .. 8q+3 (8q+4 .. 8q+7).
+  const int tr_off = (8 * q + (n >> 2)) * DROW + (n & 3) * 8;
+  const int ar_off = (8 * (n >> 2) + (n & 3)) * DROW + 16 * q;  // row of the lane's A operand in half 0 (half 1: + 4)
+  auto compute = [&](int tile, int b, uint32_t(&pr)[8]) {
+    // B operand of dW_in += dz^T pre_z (K = the 32 rows): rows 8q .. 8q+7 of channel col + j
+    u32x4 bop[2];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int s = 0; s < N32; ++s) {
-      const u32x4 ar = *reinterpret_cast<const u32x4*>(&dzr[b][n * DROW + (32 * s + 8 * q) * 2]);
+      for (int h = 0; h < 4; ++h)
+        bop[j][h] = __builtin_amdgcn_perm(pr[2 * h + 1], pr[2 * h], j ? 0x07060302u : 0x05040100u);
+    load_pre(tile + NBUF, pr);
+    __builtin_amdgcn_sched_barrier(0);
+    // dpre_z = dz W_in: half h's product row 4a + e is tile row 8a + 4h + e, so the lane ends
+    // with its own rows 8q + 4h .. +3
+    f32x4 acc[2][2];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] = Mma32<T>::run(ar, wop[s][j], acc[j]);
-    }
-    // lane (q, n) now holds rows 4q .. 4q+3 of channels col .. col+3
-    const int toff = (tile - tile0) * 16 * K * 2;
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = tile * 16 + 4 * q + i;
-      const u32x2 o = {pack2<T>(acc[0][i], acc[1][i]), pack2<T>(acc[2][i], acc[3][i])};
-      bstore64<true>(o, rd, chv && tile < tile1 && m < M ? lane_off + toff + i * K * 2 : kProjOob);
-    }
-    // dW_in += dz^T pre_z: A = dz^T (ranks 16c + n, rows 4q .. 4q+3), B = pre_z rows 4q .. 4q+3 of channel col + j
-    u32x2 bop[4];
+      for (int j = 0; j < 2; ++j) acc[h][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      bop[j][0] = elem16x2(pr[0], j) | (elem16x2(pr[1], j) << 16);
-      bop[j][1] = elem16x2(pr[2], j) | (elem16x2(pr[3], j) << 16);
-    }
+    for (int s = 0; s < N32; ++s)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u32x4 ar = *reinterpret_cast<const u32x4*>(&dzl[b][ar_off + 4 * h * DROW + 64 * s]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[h][j] = Mma32<T>::run(ar, wop[s][j], acc[h][j]);
+      }
+    const int toff = (tile - tile0) * 32 * K * 2;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      __builtin_amdgcn_raw_buffer_store_b32(pack2<T>(acc[i >> 2][0][i & 3], acc[i >> 2][1][i & 3]), rd,
+                                            chv ? lane_off + toff + i * K * 2 : kProjOob, 0, kNt);
 #pragma unroll
     for (int c = 0; c < NB; ++c) {
-      const u32x2 at = *reinterpret_cast<const u32x2*>(&dzt[b][(16 * c + n) * TROW + 8 * q]);
+      const u32x2 lo = lds_read_tr16(&dzl[b][tr_off + 32 * c]);
+      const u32x2 hi = lds_read_tr16(&dzl[b][tr_off + 32 * c + 4 * DROW]);
+      const u32x4 at = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) dw[c][j] = Mma16<T>::run(at, bop[j], dw[c][j]);
+      for (int j = 0; j < 2; ++j) dw[c][j] = Mma32<T>::run(at, bop[j], dw[c][j]);
     }
   };
 
   const int nt = tile1 - tile0;
-  for (int it = 0; it < nt; it += 2) {
-    // tile it from (buffer 0, pa); tile it + 1 from (buffer 1, pb)
-    load_dz(tile0 + it + 1);
-    load_pre(tile0 + it + 1, pb);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(tile0 + it, 0, pa);
-    store_dz(1);  // buffer 1 was last read before the previous barrier
-    __syncthreads();
-    if (it + 1 >= nt) break;  // uniform across the workgroup
-    load_dz(tile0 + it + 2);
-    load_pre(tile0 + it + 2, pa);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(tile0 + it + 1, 1, pb);
-    store_dz(0);
-    __syncthreads();
+  for (int it = 0; it < nt; it += NBUF) {
+#pragma unroll
+    for (int u = 0; u < NBUF; ++u) {
+      if (it + u >= nt) break;  // uniform across the workgroup
+      load_dz(tile0 + it + u + 2, sv[u & 1]);
+      compute(tile0 + it + u, u & 1, pre[u]);
+      store_dz(1 - (u & 1), sv[1 - (u & 1)]);  // last read before the previous barrier
+      __syncthreads();
+    }
   }
 
-  // dW_in partial of this run: rank 16c + 4q + i, channels col .. col+3
+  // dW_in partial of this run: rank 16c + 4q + i, channels col, col+1
   const rsrc_t rpart = make_rsrc_wave<kProjOob>(a.part + (int64_t)run * N * K, (int64_t)N * K * 4);
 #pragma unroll
   for (int c = 0; c < NB; ++c)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int rk = 16 * c + 4 * q + i;
-      const u32x4 v = {__float_as_uint(dw[c][0][i]), __float_as_uint(dw[c][1][i]), __float_as_uint(dw[c][2][i]),
-                       __float_as_uint(dw[c][3][i])};
-      bstore128<false>(v, rpart, chv && rk < N ? (rk * K + col) * 4 : kProjOob);
+      bstore64<false>(u32x2{__float_as_uint(dw[c][0][i]), __float_as_uint(dw[c][1][i])}, rpart,
+                      chv && rk < N ? (rk * K + col) * 4 : kProjOob);
     }
 }
 
 // ------------------------------------------------------------------ host
 namespace {
-
-constexpr int kProjBwdTargetBlocks = 512;
 
 int nb_of(int64_t N) { return (int)((N + 15) / 16); }
 
@@ -358,16 +383,31 @@ struct ProjBwdPlan {
   int ncg, nrun, seg;
 };
 
+// Runs of 32-row tiles: of the run lengths that fill an eighth of the chip's 256
+// workgroups (one to a CU) to four rounds of them, the one with the least time by a model of a
+// round's start, its tiles, and the fp32 dW_in partial each run writes and the
+// reduction reads.
 ProjBwdPlan bwd_plan(const ProjProblem& p) {
+  constexpr int64_t kSlots = 256;
   ProjBwdPlan pl;
-  const int64_t ntile = (p.M + 15) / 16;
+  const int64_t ntile = (p.M + 31) / 32;
   pl.ncg = (int)((p.K + 255) / 256);
-  int64_t nrun = (kProjBwdTargetBlocks + pl.ncg - 1) / pl.ncg;
-  if (nrun > ntile) nrun = ntile;
-  if (nrun < 1) nrun = 1;
-  const int64_t seg = (ntile + nrun - 1) / nrun;
-  pl.seg = (int)seg;
-  pl.nrun = (int)((ntile + seg - 1) / seg);
+  const double tile_us = 1.2, part_us = (double)p.G * p.R * p.K * 8 / 5e6;
+  int64_t best = ntile;
+  double best_us = -1;
+  for (int64_t slots = kSlots / 8; slots <= 4 * kSlots; slots *= 2) {
+    const int64_t runs = slots / pl.ncg;
+    if (runs < 1) continue;
+    const int64_t seg = (ntile + runs - 1) / runs, nrun = (ntile + seg - 1) / seg;
+    const double rounds = slots <= kSlots ? 1 : (double)slots / kSlots;
+    const double us = rounds * (4.0 + seg * tile_us) + nrun * part_us;
+    if (best_us < 0 || us < best_us) {
+      best = seg;
+      best_us = us;
+    }
+  }
+  pl.seg = (int)best;
+  pl.nrun = (int)((ntile + best - 1) / best);
   return pl;
 }
 
@@ -412,10 +452,12 @@ hipError_t launch_bwd(const ProjProblem& p) {
   a.ncg = pl.ncg;
   a.seg = pl.seg;
   a.nblk = pl.ncg * pl.nrun;
-  switch (nb_of(a.N)) {
-#define DC_PB(NBV) \
-  case NBV: proj_bwd<T, NBV><<<a.nblk, 256, 0, p.stream>>>(a); break;
-    DC_PB(1) DC_PB(2) DC_PB(3) DC_PB(4) DC_PB(5) DC_PB(6) DC_PB(7) DC_PB(8)
+  switch (nb_of(a.N) * 8 + (int)p.G) {
+#define DC_PB(NBV, NGV) \
+  case NBV * 8 + NGV: proj_bwd<T, NBV, NGV><<<a.nblk, 512, 0, p.stream>>>(a); break;
+#define DC_PBG(NBV) DC_PB(NBV, 1) DC_PB(NBV, 2) DC_PB(NBV, 3) DC_PB(NBV, 4)
+    DC_PBG(1) DC_PBG(2) DC_PBG(3) DC_PBG(4) DC_PBG(5) DC_PBG(6) DC_PBG(7) DC_PBG(8)
+#undef DC_PBG
 #undef DC_PB
     default: return hipErrorInvalidValue;
   }
@@ -434,9 +476,9 @@ bool proj_shape_ok(const ProjProblem& p) {
   // row indices (tiles of 16, blocks of 64 rows) are int: m0 + 64 stays in range
   if (p.M > INT32_MAX - 64) return false;
   // byte offsets within int32, below the out-of-range offset
-  if ((int64_t)N * p.K * 4 >= kProjOob || 16 * p.K * 2 >= kProjOob) return false;
+  if ((int64_t)N * p.K * 4 >= kProjOob || 32 * p.K * 2 >= kProjOob) return false;
   const ProjBwdPlan pl = bwd_plan(p);
-  return (int64_t)pl.seg * 16 * p.K * 2 + 16 * p.K * 2 < kProjOob;
+  return (int64_t)(pl.seg + 3) * 32 * p.K * 2 < kProjOob;
 }
 
 int64_t proj_bwd_ws_bytes(const ProjProblem& p) {
