@@ -584,11 +584,16 @@ LrF32mArgs make_f32m_args(const LrProblem& p) {
   a.RK = (int)p.R + (p.static_w ? 1 : 0);
   a.residual = p.residual;
   a.nch = (int)((p.D + 63) / 64);
-  // runs of about 8 tiles, at most 4096 wavefronts
+  // runs of about 8 tiles, at most 4096 wavefronts; a problem below 8 tiles for
+  // each of 2048 takes shorter runs instead of fewer wavefronts (a run's tiles
+  // are a serial chain that nothing else on an idle chip hides).  Forward, runs
+  // of 8 tiles -> filled: B2 T512 D256 R15 + static 16.0 -> 5.0 us, B1 T2048
+  // D2048 R16 17.5 -> 9.5, B1 T1000 D512 R15 + static W 16 56 -> 14; B4 T4096
+  // D2048 R16 keeps its plan (55 us).
   const int64_t ntile = (p.T + 15) / 16;
   const int64_t tiles = p.B * ntile * a.nch;
   int64_t waves = tiles / 8;
-  if (waves < 1) waves = 1;
+  if (waves < 2048) waves = tiles < 2048 ? tiles : 2048;
   if (waves > 4096) waves = 4096;
   int64_t seg = (tiles + waves - 1) / waves;
   if (seg < 1) seg = 1;
@@ -732,6 +737,46 @@ hipError_t lr_f32m_fwd(const LrProblem& p) {
 
 namespace {
 
+// Tap passes of a W-tap problem: one for W <= 4, else ceil(W / 4) of 2-4 taps
+// (the scatter form needs at least 2), the larger ones first: W 5 = 3 + 2,
+// 8 = 4 + 4, 9 = 3 + 3 + 3, 17 = 4 + 4 + 3 + 3 + 3, 32 = 8 x 4.
+inline int f32m_tap_passes(int W) { return W <= 4 ? 1 : (W + 3) / 4; }
+
+// Tiles per run of lr_bwd_f32m: a CU holds one of its workgroups (LDS), so a
+// launch takes ceil(workgroups / 256) rounds of a run's length each, and a few
+// workgroups past a round cost as much as a full one (B1 T8192 D768 R15 +
+// static W 8: runs of 6 tiles are 258 workgroups and took 152 us, runs of 7
+// 97 us; B8 T3000 D768 R15 + static W 2: 264 workgroups 75 us, 240 56 us).  Of
+// the run lengths that fill one to eight rounds and twice these, the one with
+// the least time by a model: per round and pass a launch's start and end (6 us)
+// and the run's tiles, and every run's dU partial written and read once (B2
+// T1024 D512 R16 W 4: 25.1 us at runs of 2 tiles, 26.7 at 1; B2 T512 D256 R15 +
+// static 20.9 at 2, 18.7 at 1).  dflt: no such length (more sequences than
+// eight rounds hold).
+int64_t f32m_bwd_run_tiles(const LrProblem& p, int64_t ntile, int64_t cols, int64_t dflt) {
+  constexpr int64_t kCus = 256;
+  const int64_t RK = p.R + (p.static_w ? 1 : 0), rank_passes = (RK + 15) / 16;
+  const double start_us = 6.0 * rank_passes * f32m_tap_passes((int)p.W);
+  const double tile_us = 0.75 * p.W * rank_passes;
+  const double part_us = (double)RK * p.W * p.D * 8 / 5e6;
+  int64_t best = dflt;
+  double best_us = -1;
+  for (int64_t rounds = 1; rounds <= 8; ++rounds) {
+    const int64_t per_seq = rounds * kCus / (p.B * cols);  // runs a sequence may take
+    if (per_seq < 1) continue;
+    const int64_t fill = (ntile + per_seq - 1) / per_seq;
+    for (int64_t seg = fill; seg <= 2 * fill; seg += fill) {
+      const int64_t runs = p.B * ((ntile + seg - 1) / seg), n = (runs * cols + kCus - 1) / kCus;
+      const double us = n * (start_us + seg * tile_us) + runs * part_us;
+      if (best_us < 0 || us < best_us) {
+        best = seg;
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
 LrF32mBwdArgs make_f32m_bwd_args(const LrProblem& p) {
   LrF32mBwdArgs a;
   a.Tn = (int)p.T;
@@ -741,10 +786,9 @@ LrF32mBwdArgs make_f32m_bwd_args(const LrProblem& p) {
   a.residual = p.residual;
   a.nch = (int)((p.D + 31) / 32);
   a.ncg = (a.nch + 7) / 8;
-  // 2048 wavefronts (2 per SIMD): runs of ceil(tiles * 8 chunks / 2048) tiles
   const int64_t ntile = (p.T + 15) / 16;
-  int64_t seg = (p.B * ntile * a.ncg * 8 + 2047) / 2048;
-  if (seg < 2) seg = 2;
+  int64_t seg = f32m_bwd_run_tiles(p, ntile, a.ncg, (p.B * ntile * a.ncg + 255) / 256);
+  if (seg < 1) seg = 1;
   if (seg > ntile) seg = ntile;
   const int64_t cap = f32m_bwd_max_run_tiles(p);  // >= 1 (lr_f32m_bwd_ok)
   if (seg > cap) seg = cap;
@@ -765,10 +809,6 @@ LrF32mBwdArgs make_f32m_bwd_args(const LrProblem& p) {
 struct F32mWs {
   int64_t dz_off, du_off, total;
 };
-// Tap passes of a W-tap problem: one for W <= 4, else ceil(W / 4) of 2-4 taps
-// (the scatter form needs at least 2), the larger ones first: W 5 = 3 + 2,
-// 8 = 4 + 4, 9 = 3 + 3 + 3, 17 = 4 + 4 + 3 + 3 + 3, 32 = 8 x 4.
-inline int f32m_tap_passes(int W) { return W <= 4 ? 1 : (W + 3) / 4; }
 inline int f32m_pass_taps(int W, int tp) {
   const int n = f32m_tap_passes(W), base = W / n;
   return tp < W % n ? base + 1 : base;
