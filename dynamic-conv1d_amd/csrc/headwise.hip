@@ -134,18 +134,41 @@ int unroll_of(int W) { return W >= 4 ? W : W * (4 / W); }
 
 bool aligned(const void* p, int a) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 
+// The run length seg, or up to a quarter longer (`one_wg`: at least one step)
+// where that keeps the launch within `fill` workgroups of 4 runs.  The
+// last run of every sequence is shorter, so seg rows to a run may give a few
+// workgroups more than are resident at once, and these cost a large part of
+// another round.  Forward + backward, W 4 and bf16 unless stated, before and
+// now: B2 T8192 D1280 head size 1 64 + 162 -> 50 + 122 us (258 -> 238
+// workgroups), head size 32 24 + 47 -> 20 + 35; B2 T5185 D3200 head size 1
+// fp32 222 + 461 -> 187 + 335; B8 T2288 D2816 W 6 head size 1 217 + 484 -> 159
+// + 375.  Where a CU holds one workgroup (more than 256 registers: the
+// backward, and the forward from W 6 on) a step more pays at any length: B3
+// T2048 D1912 W 8 forward 84.5 -> 59.6 us at four steps of 8 rows instead of
+// three; with two and more to a CU runs of three steps stretched to four do not
+// (B1 T2048 D1408 fp32 forward 17.2 -> 18.4 us).
+int64_t fit_run(int64_t B, int64_t T, int64_t cols, int64_t seg, int64_t step, int64_t fill, bool one_wg) {
+  int64_t slack = seg / 4;
+  if (one_wg && slack < step) slack = step;
+  for (int64_t s = seg; s <= seg + slack; s += step)
+    if ((B * ((T + s - 1) / s) + 3) / 4 * cols <= fill) return s;
+  return seg;
+}
+
 // Run length: aim for `target_waves` wavefronts in total (1024 = one per
 // SIMD of the 256 CUs: with the next chunk always in flight, fewer and longer
 // runs measured faster than more, shorter ones), at least 4 rows, a multiple
 // of the unroll.  Small problems get short runs so that the grid still covers
 // the CUs: configs[0] (B2 T1024 D512, head size 1, fp32) forward 10.3 -> 6.4 us
 // and backward 22.4 -> 13.0 us with a minimum of 4 rows instead of 16.
-int choose_seg(int64_t B, int64_t T, int64_t nvg, int W, int target_waves) {
+int choose_seg(int64_t B, int64_t T, int64_t nvg, int W, int target_waves, bool bwd) {
   const int u = unroll_of(W);
   int64_t seg = (B * T * nvg + target_waves - 1) / target_waves;
   if (seg < 4) seg = 4;
   seg = (seg + u - 1) / u * u;
-  if (seg > T) seg = (T + u - 1) / u * u;
+  const int64_t whole = (T + u - 1) / u * u;
+  if (seg > whole) seg = whole;
+  seg = fit_run(B, T, nvg, seg, u, target_waves / 4, bwd || W >= 6);
   return (int)seg;
 }
 
@@ -167,7 +190,7 @@ HwPlan make_plan(const HwProblem& p, bool bwd) {
   a.hs_shift = ilog2(hs);
   a.nvc = (int)(p.D / VEC);
   a.nvg = (a.nvc + 63) / 64;
-  a.seg = choose_seg(p.B, p.T, a.nvg, (int)p.W, 1024);
+  a.seg = choose_seg(p.B, p.T, a.nvg, (int)p.W, 1024, bwd);
   // a run's buffer resources span (seg + kHwSlackRows) rows at most kHwRunBytes
   const int u = unroll_of((int)p.W);
   const int64_t seg_cap = (kHwRunBytes / max_row_bytes(p) - kHwSlackRows) / u * u;
