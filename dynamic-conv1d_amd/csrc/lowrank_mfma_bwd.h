@@ -64,7 +64,7 @@ struct Pair {
 // A lane's two channels of one dx row as the passes keep them: the output type
 // (DxVec<T, false>), or past four passes (two that split the ranks) an fp32
 // accumulator in the workspace (DxVec<T, true>), which the last pass rounds to
-// dx once (more passes rounded in 16 bits each drift past the north-star bar).
+// dx once (more passes rounded in 16 bits each drift past the 2e-2 elementwise bar).
 template <typename T, bool F32> struct DxVec {
   typedef uint32_t type;
   static constexpr int ES = 2;
