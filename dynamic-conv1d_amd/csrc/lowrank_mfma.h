@@ -232,10 +232,15 @@ struct ZRaw {
 // dx of the backward over all kernel ranks in one launch (lowrank_mfma_dx.hip;
 // the passes of ranks then form dz and dU only).
 template <typename T>
-hipError_t lr_dx_mfma_launch(const LrProblem* p, int G, const void* const* z, int zld);
+hipError_t lr_dx_mfma_launch(const LrProblem* p, int G, const void* const* z, int zld, void* const* acc);
 // Its shapes: the packed U operands of all taps and ranks in one workgroup's LDS
 // (W x 32-rank chunks x 8 KiB, at most 128 KiB), the look-ahead in one lane group.
-inline bool lr_dx_split_shape(int64_t RK, int64_t W) { return W <= 8 && RK <= 128 && W * ((RK + 31) / 32) <= 16; }
+// (two launches of taps over an fp32 accumulator at W 9-16 and kernel rank <= 64)
+inline bool lr_dx_two_passes(int64_t W) { return W > 8; }
+inline bool lr_dx_split_shape(int64_t RK, int64_t W) {
+  if (lr_dx_two_passes(W)) return W <= 16 && RK <= 64;
+  return RK <= 128 && W * ((RK + 31) / 32) <= 16;
+}
 
 inline bool aligned_to(const void* p, int a) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 

@@ -397,13 +397,17 @@ inline int bwd_rank_passes(const LrProblem& p) {
 constexpr int kBwdMaxBf16DxPasses = 4;
 constexpr int kBwdMaxBf16DxRankPasses = 2;
 // Passes of ranks with dy in [B, T, D] whose dx fits one launch
-// (lr_dx_split_shape: W <= 8 up to kernel rank 64, W 5 / 4 up to 96 / 128): the
+// (lr_dx_split_shape: W <= 8 up to kernel rank 64, W 5 / 4 up to 96 / 128) or,
+// with dy in either layout, two (W 9-16 up to 64, over the fp32 accumulator): the
 // passes form dz and dU only (DXM 3) and lr_dx_t32 forms dx over all ranks and
 // taps in one launch, rounded once (no fp32 accumulator).  Passes of taps alone
 // (two rank chunks above W 4) keep dx: split off it measured 160 -> 166 us at B4
 // T4096 D2048 R31 + static W 8.
 inline bool bwd_dx_split(const LrProblem& p) {
-  return bwd_rank_split(p) && lr_dx_split_shape(p.R + (p.static_w ? 1 : 0), p.W) && p.yhd() == p.D;
+  const int64_t hd = p.yhd();
+  // head-major dy: two launches only, where a chunk's heads fit one resource
+  const bool dy_ok = hd == p.D || (lr_dx_two_passes(p.W) && (127 / hd + 2) * (p.T + 64) * hd * 2 < kMaxSeqBytes);
+  return bwd_rank_split(p) && lr_dx_split_shape(p.R + (p.static_w ? 1 : 0), p.W) && dy_ok;
 }
 // The workspace keeps room for the accumulator whether or not dx is split off:
 // the size queries do not see dy's layout, on which the split depends.
@@ -777,7 +781,13 @@ hipError_t launch_bwd(const LrProblem* p, int G) {
   if (dxs) {
     const void* zs[kMaxGroups];
     for (int g = 0; g < G; ++g) zs[g] = a.grp[g].z;
-    if ((e = lr_dx_mfma_launch<T>(p, G, zs, a.zld)) != hipSuccess) return e;
+    void* acc[kMaxGroups];
+    for (int g = 0; g < G; ++g) acc[g] = (char*)p[g].ws + w.dxf_off;
+    if ((e = lr_dx_mfma_launch<T>(p, G, zs, a.zld, acc)) != hipSuccess) return e;
+    // the rows that the second launch's taps do not reach, from the accumulator
+    if (lr_dx_two_passes(p[0].W) &&
+        (e = launch_dx_round_tail<T>(p, G, w.dxf_off, (int)(p[0].W - p[0].W / 2))) != hipSuccess)
+      return e;
   }
   // The last pass stores dx rows 0 .. T-1-kofs of its taps kofs ..; the rows
   // after those (no terms of its taps) are rounded from the accumulator here

@@ -269,7 +269,14 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_fwd_t32(LrArgs a)
 // group 3's open rows wait one tile in fp32 (carry).  The tile after a run closes
 // its last rows.  z is read as z_eff rows of 32 NC ranks (grp.z, zld; static column
 // included), grp.x is dy, grp.y dx (rows yhd apart).
-template <typename T, int W, int NC>
+//
+// M: taps past one launch's operands take two (kernel rank 33-64 at W 9-16), over
+// an fp32 accumulator (grp.zeff, rows of D): M 1 stores it, M 2 (taps kofs .., its
+// rows kofs earlier) adds it and stores dx, rounded once; dx's last kofs rows, which
+// get no terms of M 2's taps, are left to the caller.  Against passes of 32 ranks x 4
+// taps that each added dx into the accumulator, whole backward at B4 T4096 D2048
+// bf16: R40 W 12 616 -> 382 us, R64 W 16 890 -> 534 us.
+template <typename T, int W, int NC, int M = 0>
 __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) {
   constexpr int NWV = t32_wg_waves(W, NC);
   constexpr int NO = W > 1 ? W - 1 : 1;  // open rows of a group (none at W 1)
@@ -296,16 +303,30 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) 
   if (sg >= a.nseg) return;
   const T32Run run(a, sg);
   const int rb = run.rb, tile0 = run.tile0, tile1 = run.tile1, ntile = (Tn + 31) >> 5;
-  const int dyrowb = a.xld * 2, dxrowb = a.yhd * 2, zld = a.zld;
-  const rsrc_t rdy = run_rsrc(dy + run.rrow * a.xld, Tn - rb, dyrowb);
+  // dy is [B, T, D] (hd == D), with M also head-major [B, D/hd, T, hd]: the resource then
+  // spans the chunk's heads (loads check the row against T)
+  const int hd = M ? a.zrp : a.xld, yh = M ? dl / hd : 0, yh0 = M ? chunk * 128 / hd : 0;
+  const int yhl = M ? min(chunk * 128 + 127, D - 1) / hd : 0;
+  const int dyrowb = hd * 2, dxrowb = a.yhd * 2, zld = a.zld;
+  const rsrc_t rdy = run_rsrc(dy + run.row0 * a.xld + ((int64_t)yh0 * Tn + rb) * hd,
+                              (int64_t)(yhl - yh0) * Tn + Tn - rb, dyrowb);
   const rsrc_t rdx = run_rsrc(dx + run.rrow * a.yhd, Tn - rb, dxrowb);
   const rsrc_t rz = run_rsrc(z + run.rrow * zld, Tn - rb, zld * 2);
-  const int dylane = chv ? (8 * q * a.xld + dl) * 2 : kOobLane;
+  const int dylane = chv ? (((yh - yh0) * Tn + 8 * q) * hd + dl - yh * hd) * 2 : kOobLane;
   const int dxlane = chv ? (8 * q * a.yhd + dl) * 2 : kOobLane;
   const int below = ((lane + 16) & 63) << 2;  // ds_bpermute byte index of the group below
   const int zrow = 8 * (n >> 2) + (n & 3);
   const float res = a.residual ? 1.f : 0.f;
   const bool top = q == 3;
+  const int accrowb = D * 4, kofs = M == 2 ? a.kofs : 0;
+  const rsrc_t racc = run_rsrc(reinterpret_cast<float*>(gp->zeff) + run.rrow * D, Tn - rb, M ? accrowb : 0);
+  // M: the row of the resources that the lane's row i of a tile closes as (-1: none)
+  auto acc_row = [&](int tile, int i) {
+    const bool before = top && W > 1 && i >= kFirstOpen;  // group 3's open rows close a tile late
+    const int t = (before ? tile - 1 : tile) * 32 + 8 * q + i;
+    const bool ok = chv && (before ? tile > tile0 : tile < tile1) && t >= kofs && t < Tn;
+    return ok ? t - kofs - rb : -1;
+  };
 
   float carry[4][2][NO];  // group 3's open rows of the tile before (the run's first tile stores none)
 #pragma unroll
@@ -320,13 +341,24 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) 
     const int toff = live ? (tile * 32 - rb) * dyrowb : kOobTile;
     u32x4 dyr[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) dyr[i] = bload128(rdy, dylane + toff + i * dyrowb);
+    for (int i = 0; i < 8; ++i)
+      dyr[i] = bload128(rdy, M && tile * 32 + 8 * q + i >= Tn ? kOobTile : dylane + toff + i * dyrowb);
     u32x4 zc[2][NC];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int c = 0; c < NC; ++c)
         zc[h][c] = bload128(rz, live ? (tile * 32 + zrow + 4 * h - rb) * zld * 2 + (32 * c + 8 * q) * 2 : kOobTile);
+    u32x4 acc[M ? 8 : 1][2];  // the accumulator's rows (M 1: to store)
+    if constexpr (M == 2) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int r = acc_row(tile, i);
+          acc[i][h] = bload128(racc, r >= 0 ? r * accrowb + dl * 4 + 16 * h : kOobTile);
+        }
+    }
     u32x4 out[8];
 #pragma unroll
     for (int h4 = 0; h4 < 4; ++h4) {
@@ -365,10 +397,41 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) 
           }
         }
       }
+      if constexpr (M == 1) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) out[i][h4] = pack2<T>(v[0][i], v[1][i]);
-      end_pair(out, h4);
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+          for (int jj = 0; jj < 2; ++jj) {
+            uint32_t o = __float_as_uint(v[jj][i]);
+            asm volatile("" : "+v"(o) : : "memory");  // as end_pair
+            acc[i][h4 >> 1][2 * (h4 & 1) + jj] = o;
+          }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if constexpr (M == 2) {
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj) v[jj][i] += __uint_as_float(acc[i][h4 >> 1][2 * (h4 & 1) + jj]);
+          }
+          out[i][h4] = pack2<T>(v[0][i], v[1][i]);
+        }
+        end_pair(out, h4);
+      }
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (M != 0) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = acc_row(tile, i);
+        if constexpr (M == 2) {
+          bstore128<true>(out[i], rdx, r >= 0 ? r * dxrowb + dl * 2 : kOobTile);
+        } else {
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            bstore128<false>(acc[i][h], racc, r >= 0 ? r * accrowb + dl * 4 + 16 * h : kOobTile);
+        }
+      }
+      continue;
     }
     const int cur_off = tile < tile1 ? dxlane + (tile * 32 - rb) * dxrowb : kOobTile;
     const int prev_off = tile > tile0 ? dxlane + ((tile - 1) * 32 - rb) * dxrowb : kOobTile;
@@ -384,6 +447,6 @@ template <typename T>
 hipError_t lr_fwd_t32_launch(const LrArgs& a, int W, int NC, hipStream_t stream);
 // dx launch on lr_dx_t32.
 template <typename T>
-hipError_t lr_dx_t32_launch(const LrArgs& a, int W, int NC, hipStream_t stream);
+hipError_t lr_dx_t32_launch(const LrArgs& a, int W, int NC, int M, hipStream_t stream);
 
 }  // namespace dc

@@ -28,6 +28,11 @@ CASES = (
     + [(2, 100, 72, R, W, st, bf16) for R, W, st in ((40, 3, True), (63, 4, True), (64, 4, True), (127, 2, True),
                                                         (63, 5, True), (40, 6, False), (63, 8, True), (80, 5, True),
                                                         (64, 8, False), (127, 4, True), (96, 1, False))]
+    # dx in two launches of taps over an fp32 accumulator: sequences shorter than the second's
+    # first tap, of whole tiles, and off them
+    + [(2, T, D, R, W, st, bf16) for T, D, R, W, st in ((5, 40, 40, 12, False), (64, 136, 63, 9, True),
+                                                          (33, 264, 64, 16, False), (100, 72, 50, 13, True))]
+    + [(1, 35050, 136, 40, 10, True, fp16)]
     # its runs of tiles: the dx launch's carry over tiles, the tile after a run
     + [(1, 70100, 136, 63, 4, True, bf16), (1, 70100, 136, 40, 8, True, fp16)]
     # passes of taps (dx of the earlier passes added) at one and two rank chunks, rows 32 apart from the halo
