@@ -272,8 +272,14 @@ int dc_lowrank_path(int64_t B, int64_t T, int64_t D, int64_t R, int64_t W, int d
   return dc::lr_path(p, bwd != 0);
 }
 
-int64_t dc_lowrank_plan_ranges(int64_t B, int64_t T, int64_t D, int64_t R, int64_t W, int dtype, int has_static,
-                               int bwd, int64_t* out, int64_t max_pairs) {
+// dc_lowrank_plan_ranges for one group of a grouped call: rows of x / dx x_ld /
+// dx_ld elements apart, y (dy) head-major when y_hd > 0, and a workspace of
+// ws_bytes, whose pairs (the end of the dU partials and of the whole workspace,
+// each with what there is room for) come with the backward's.  A test hook that
+// the header does not declare.
+int64_t dc_lowrank_strided_plan_ranges(int64_t B, int64_t T, int64_t D, int64_t R, int64_t W, int dtype, int has_static,
+                                       int bwd, int64_t x_ld, int64_t dx_ld, int64_t y_hd, int64_t ws_bytes,
+                                       int64_t* out, int64_t max_pairs) {
   int s = check_lowrank(B, T, D, R, W, dtype, has_static != 0);
   if (s != DC_OK) return s;
   if (max_pairs < 0 || (max_pairs > 0 && !out)) return DC_ERR_NULL;
@@ -284,15 +290,23 @@ int64_t dc_lowrank_plan_ranges(int64_t B, int64_t T, int64_t D, int64_t R, int64
   p.x = p.z = p.U = p.dy = kAligned;
   p.y = p.dx = p.dz = p.dU = (void*)kAligned;
   p.ws = (float*)kAligned;
+  p.ws_bytes = ws_bytes;
   p.static_w = has_static ? kAligned : nullptr;
   p.dstatic_w = has_static ? (void*)kAligned : nullptr;
   p.B = B; p.T = T; p.D = D; p.R = R; p.W = W; p.dtype = dtype; p.residual = 1;
+  p.x_ld = x_ld; p.dx_ld = dx_ld; p.y_hd = y_hd;
   if (dc::lr_path(p, bwd != 0) == DC_PATH_GENERIC) return 0;  // generic kernels: plain pointers
   dc::RangeAudit audit{out, max_pairs, 0};
   dc::g_range_audit = &audit;
   const hipError_t e = bwd ? dc::lr_bwd(&p, 1) : dc::lr_fwd(&p, 1);
   dc::g_range_audit = nullptr;
   return e == hipSuccess ? audit.n : DC_ERR_LAUNCH;
+}
+
+int64_t dc_lowrank_plan_ranges(int64_t B, int64_t T, int64_t D, int64_t R, int64_t W, int dtype, int has_static,
+                               int bwd, int64_t* out, int64_t max_pairs) {
+  const int64_t ws = bwd ? dc_lowrank_bwd_ws_bytes(B, T, D, R, W, dtype, has_static) : 0;
+  return dc_lowrank_strided_plan_ranges(B, T, D, R, W, dtype, has_static, bwd, 0, 0, 0, ws < 0 ? 0 : ws, out, max_pairs);
 }
 
 int64_t dc_lowrank_bwd_ws_bytes(int64_t B, int64_t T, int64_t D, int64_t R, int64_t W, int dtype,

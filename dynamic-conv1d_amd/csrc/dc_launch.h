@@ -50,6 +50,7 @@ struct LrProblem {
   void* dU;
   void* dstatic_w;
   float* ws;
+  int64_t ws_bytes;       // bytes of ws (read by the range audit alone)
   // Padded z_eff [B*T, RP] of z's type (RP = lr_bwd_zrow), or null: the forward
   // writes it, the backward reads it instead of building it (lowrank only).
   void* zeff;
@@ -88,6 +89,16 @@ struct LrProblem {
 // static_w and the x / dx row strides; pointers differ.  The backward's
 // workspace is G consecutive per-group workspaces.
 constexpr int kMaxGroups = 4;
+
+// The problem as the workspace size query sees it: contiguous x, dx and dy.  The
+// matrix-core backwards write one fp32 dU partial per run, and a run's buffer
+// resources hold fewer rows of a wider x or dx: such a call can have more runs
+// than the query's plan, and so than its workspace has dU slots.  It then runs
+// in parts (DuParts).
+inline LrProblem contiguous_problem(LrProblem p) {
+  p.x_ld = p.dx_ld = p.y_hd = 0;
+  return p;
+}
 
 bool lr_mfma_ok(const LrProblem& p, bool bwd);
 // dc_path code of the kernels lr_fwd / lr_bwd run for one problem p.
@@ -157,5 +168,27 @@ struct PartialReduce {
   void* out;
 };
 hipError_t reduce_partials_multi(const PartialReduce* r, int n, int dtype, hipStream_t stream);
+
+// The parts of a backward whose runs exceed the workspace's dU slots: a part's
+// launches take runs run0 .. run0 + n - 1 and write their partials to slots
+// slot0 .. slot0 + n - 1; before the next part, a fold sums the slots so far into
+// slot 0, in fp32 and in a fixed order.  One part, and no fold, unless a row
+// stride caps the runs.
+//   DuParts t(nruns, slots);
+//   for (;; t.next()) { launches; if (!t.more()) break; fold }
+struct DuParts {
+  int nruns, slots, run0 = 0, slot0 = 0, n;
+  DuParts(int nruns, int slots) : nruns(nruns), slots(slots), n(nruns < slots ? nruns : slots) {}
+  bool more() const { return run0 + n < nruns; }
+  int used() const { return slot0 + n; }  // slots that hold sums after this part
+  void next() {
+    run0 += n;
+    slot0 = 1;
+    const int left = nruns - run0;
+    n = left < slots - 1 ? left : slots - 1;
+  }
+};
+// dU slots for the runs of the contiguous plan (run_tiles each): at least two where more runs can arise.
+inline int du_slots(int nruns, int run_tiles) { return nruns > 1 || run_tiles < 2 ? nruns : 2; }
 
 }  // namespace dc

@@ -429,6 +429,7 @@ hipError_t launch_f32(const LrProblem& p, bool bwd) {
     audit_range(lr_sw_bytes(p.static_w != nullptr, W, a.D, 4), kOobLane);
     const int64_t rows[4] = {(int64_t)a.xld * 4, (int64_t)a.yhd * 4, (int64_t)p.dxld() * 4, (int64_t)a.R * 4};
     for (int64_t rowb : rows) audit_range((int64_t)a.Tn * rowb, kMaxSeqBytes - kSeqSlackRows * rowb);
+    if (bwd) audit_range(f32_ws(p, a).total, p.ws_bytes);
     return hipSuccess;
   }
   if (!bwd) {

@@ -223,7 +223,8 @@ struct LrF32mBwdArgs {
   int seg;   // 16-row tiles per run
   int nspb;  // runs per sequence
   int nseg;  // B * nspb
-  int nblk;  // ncg * nseg
+  int sp0;   // first run of the launch; its dU partial is part_du's first
+  int nblk;  // ncg * runs of the launch (nseg, or a part: DuParts)
   int xld, dxld;  // row strides of x and dx (elements)
   int yhd;        // dy layout: D ([B, T, D]) or the head dim of [B, D/yhd, T, yhd] (yhd % 32 == 0)
   int rofs;       // first kernel rank of this pass (0, or 16 for the second of two)
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(512) void lr_bwd_f32m(const float* __restrict__ x, 
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int q = lane >> 4, n = lane & 15;
   const int lb = xcd_remap(blockIdx.x, a.nblk);
-  const int cg = lb % a.ncg, s = lb / a.ncg;
+  const int cg = lb % a.ncg, du_slot = lb / a.ncg, s = a.sp0 + du_slot;
   const int chunk = cg * NCW + wave;
   const int D = a.D, Tn = a.Tn, R = a.R, RK = a.RK, rofs = ACC ? a.rofs : 0, kofs = ACC ? a.kofs : 0;
   const int uld = a.uld;
@@ -542,7 +543,7 @@ __global__ __launch_bounds__(512) void lr_bwd_f32m(const float* __restrict__ x, 
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int rk = rofs + 4 * q + r;  // kernel rank (this pass's 16)
-        if (rk < RK && chv) part_du[((int64_t)s * RK + rk) * uld + (int64_t)k * D + col + jj] = du[k][jj][r];
+        if (rk < RK && chv) part_du[((int64_t)du_slot * RK + rk) * uld + (int64_t)k * D + col + jj] = du[k][jj][r];
       }
 }
 
@@ -795,6 +796,7 @@ LrF32mBwdArgs make_f32m_bwd_args(const LrProblem& p) {
   a.seg = (int)seg;
   a.nspb = (int)((ntile + seg - 1) / seg);
   a.nseg = (int)(p.B * a.nspb);
+  a.sp0 = 0;
   a.nblk = a.nseg * a.ncg;
   a.xld = (int)p.xld();
   a.dxld = (int)p.dxld();
@@ -806,19 +808,24 @@ LrF32mBwdArgs make_f32m_bwd_args(const LrProblem& p) {
   return a;
 }
 
-struct F32mWs {
-  int64_t dz_off, du_off, total;
-};
 inline int f32m_pass_taps(int W, int tp) {
   const int n = f32m_tap_passes(W), base = W / n;
   return tp < W % n ? base + 1 : base;
 }
 
-F32mWs f32m_ws(const LrProblem& p, const LrF32mBwdArgs& a) {
+// Workspace: [dz partials: tap passes x ncg x BT x R][dU partials: one RK x W*D
+// slot per run of the contiguous problem (du_slots)].
+struct F32mWs {
+  int64_t dz_off, du_off, total;
+  int slots;
+};
+F32mWs f32m_ws(const LrProblem& p) {
+  const LrF32mBwdArgs a = make_f32m_bwd_args(contiguous_problem(p));
   F32mWs w;
+  w.slots = du_slots(a.nseg, a.seg);
   w.dz_off = 0;
   w.du_off = ((int64_t)f32m_tap_passes((int)p.W) * a.ncg * a.BT * a.R * 4 + 255) / 256 * 256;
-  w.total = w.du_off + (int64_t)a.nseg * a.RK * p.W * p.D * 4;
+  w.total = w.du_off + (int64_t)w.slots * a.RK * p.W * p.D * 4;
   return w;
 }
 
@@ -863,33 +870,43 @@ hipError_t launch_f32m_taps(const LrProblem& p, const LrF32mBwdArgs& a, const fl
 }
 
 hipError_t launch_f32m_bwd(const LrProblem& p) {
-  const LrF32mBwdArgs a = make_f32m_bwd_args(p);
-  const F32mWs w = f32m_ws(p, a);
+  LrF32mBwdArgs a = make_f32m_bwd_args(p);
+  const F32mWs w = f32m_ws(p);
   float* pdz = (float*)((char*)p.ws + w.dz_off);
   float* pdu = (float*)((char*)p.ws + w.du_off);
   const int ntp = f32m_tap_passes((int)p.W);
   const int64_t dz_slot = (int64_t)a.ncg * a.BT * a.R;  // one tap pass's dz partials
-  hipError_t e;
-  for (int tp = 0, kofs = 0; tp < ntp; kofs += f32m_pass_taps((int)p.W, tp), ++tp) {
-    const int wq = f32m_pass_taps((int)p.W, tp);
-    LrF32mBwdArgs b = a;
-    b.kofs = kofs;
-    const float* U = (const float*)p.U + (int64_t)kofs * p.D;
-    const float* sw = p.static_w ? (const float*)p.static_w + (int64_t)kofs * p.D : nullptr;
-    float* dz_t = pdz + tp * dz_slot;
-    float* du_t = pdu + (int64_t)kofs * p.D;
-    switch (wq) {
-      case 2: e = launch_f32m_taps<2>(p, b, U, sw, dz_t, du_t); break;
-      case 3: e = launch_f32m_taps<3>(p, b, U, sw, dz_t, du_t); break;
-      case 4: e = launch_f32m_taps<4>(p, b, U, sw, dz_t, du_t); break;
-      default: e = hipErrorInvalidValue; break;
-    }
-    if (e != hipSuccess) return e;
-  }
   const int64_t WD = p.W * p.D, RKWD = (int64_t)a.RK * WD;
+  hipError_t e;
+  DuParts t(a.nseg, w.slots);
+  for (;; t.next()) {
+    a.sp0 = t.run0;
+    a.nblk = t.n * a.ncg;
+    for (int tp = 0, kofs = 0; tp < ntp; kofs += f32m_pass_taps((int)p.W, tp), ++tp) {
+      const int wq = f32m_pass_taps((int)p.W, tp);
+      LrF32mBwdArgs b = a;
+      b.kofs = kofs;
+      const float* U = (const float*)p.U + (int64_t)kofs * p.D;
+      const float* sw = p.static_w ? (const float*)p.static_w + (int64_t)kofs * p.D : nullptr;
+      float* dz_t = pdz + tp * dz_slot;
+      float* du_t = pdu + t.slot0 * RKWD + (int64_t)kofs * p.D;
+      switch (wq) {
+        case 2: e = launch_f32m_taps<2>(p, b, U, sw, dz_t, du_t); break;
+        case 3: e = launch_f32m_taps<3>(p, b, U, sw, dz_t, du_t); break;
+        case 4: e = launch_f32m_taps<4>(p, b, U, sw, dz_t, du_t); break;
+        default: e = hipErrorInvalidValue; break;
+      }
+      if (e != hipSuccess) return e;
+    }
+    if (auditing()) audit_range(w.du_off + t.used() * RKWD * 4, w.total);
+    if (!t.more()) break;
+    const PartialReduce fold{pdu, RKWD, t.used(), RKWD, pdu};
+    if ((e = reduce_partials_multi(&fold, 1, kFP32, p.stream)) != hipSuccess) return e;
+  }
+  if (auditing()) audit_range(w.total, p.ws_bytes);
   const PartialReduce jobs[3] = {
-      {pdu, RKWD, a.nseg, p.R * WD, p.dU},
-      {pdu + p.R * WD, RKWD, a.nseg, p.static_w ? WD : 0, p.dstatic_w},
+      {pdu, RKWD, t.used(), p.R * WD, p.dU},
+      {pdu + p.R * WD, RKWD, t.used(), p.static_w ? WD : 0, p.dstatic_w},
       {pdz, a.BT * a.R, ntp * a.ncg, a.BT * a.R, p.dz},
   };
   return reduce_partials_multi(jobs, 3, p.dtype, p.stream);
@@ -915,7 +932,7 @@ bool lr_f32m_bwd_ok(const LrProblem& p) {
   return f32m_bwd_max_run_tiles(p) >= 1;
 }
 
-int64_t lr_f32m_ws_bytes(const LrProblem& p) { return f32m_ws(p, make_f32m_bwd_args(p)).total; }
+int64_t lr_f32m_ws_bytes(const LrProblem& p) { return f32m_ws(p).total; }
 
 hipError_t lr_f32m_bwd(const LrProblem& p) { return launch_f32m_bwd(p); }
 

@@ -27,7 +27,8 @@ struct LrBwdArgs {
   int seg;    // tiles per run
   int nspb;   // runs per sequence
   int nseg;   // B * nspb
-  int npair;  // workgroup rows: one run, one dU partial each (nseg)
+  int npair;  // workgroup rows of a launch: one run, one dU partial each (nseg, or a part of the runs: DuParts)
+  int sp0;    // first run of the launch; its dU partial is part_du's first
   int nblk;   // ncg * npair * nrp * groups
   int nblk1;  // blocks per group
   int xld;    // row stride of x (elements)

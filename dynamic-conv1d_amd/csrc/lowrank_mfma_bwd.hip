@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
   uint16_t* __restrict__ dx = reinterpret_cast<uint16_t*>(gp->dx);
   float* __restrict__ part_dz = gp->part_dz;
   float* __restrict__ part_du = gp->part_du;
-  const int cg = lb % a.ncg, sp = lb / a.ncg;
+  const int cg = lb % a.ncg, du_slot = lb / a.ncg, sp = a.sp0 + du_slot;
   const int D = a.D, Tn = a.Tn;
   const int d0 = (cg * 4 + wave) * 64;
   const int col = d0 + 4 * n;
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
   // per tap.  The resource spans the run's RK x W*D partial, so rows r >= RK fall
   // outside it (the host keeps (RK + 16) * W * D * 4 bytes below kOobLane, so no
   // offset wraps).
-  const rsrc_t rdu = make_rsrc(part_du + (int64_t)sp * a.dupr * a.uld, lr_dupart_bytes(RK, a.uld, 0, D));
+  const rsrc_t rdu = make_rsrc(part_du + (int64_t)du_slot * a.dupr * a.uld, lr_dupart_bytes(RK, a.uld, 0, D));
   const int du_lane = chv ? (4 * q * a.uld + col) * 4 : kOobLane;
 #pragma unroll
   for (int k = 0; k < W; ++k)
@@ -523,6 +523,7 @@ LrBwdArgs make_bwd_args(const LrProblem& p, int target_waves, bool split) {
   a.nspb = (int)((ntile + seg - 1) / seg);
   a.nseg = (int)(p.B * a.nspb);
   a.npair = a.nseg;
+  a.sp0 = 0;
   a.nblk = a.npair * a.ncg * a.nrp;
   a.BT = p.B * p.T;
   a.zld = a.zr = (int)p.R;
@@ -658,20 +659,24 @@ hipError_t launch_dx_round_tail(const LrProblem* p, int G, int64_t dxf_off, int 
   return hipGetLastError();
 }
 
-// Workspace: [dz partials: passes x ncg x BT x R fp32][dU partials: npair x RK
-// x W*D fp32][padded z_eff: BT x RP of z's type][past four passes, or two
-// that split the ranks: the fp32 dx accumulator, BT x D], each 256-byte aligned.  The z_eff part is reserved
-// whatever the pointers' alignment (the size query has none).
+// Workspace: [dz partials: passes x ncg x BT x R fp32][dU partials: slots x RK
+// x W*D fp32 (one per run of the contiguous problem: du_slots)][padded z_eff: BT
+// x RP of z's type][past four passes, or two that split the ranks: the fp32 dx
+// accumulator, BT x D], each 256-byte aligned.  The z_eff part is reserved
+// whatever the pointers' alignment (the size query has none, and no row strides).
 struct BwdWs {
   int64_t dz_off, du_off, zp_off, dxf_off, total;
+  int slots;  // dU partials
 };
-BwdWs bwd_ws(const LrProblem& p, const LrBwdArgs& a) {
+BwdWs bwd_ws(const LrProblem& p, bool split) {
+  const LrBwdArgs a = make_bwd_args(contiguous_problem(p), kBwdTargetWaves, split);
   BwdWs w;
+  w.slots = du_slots(a.nseg, a.seg);
   // one dz partial slot per pass of taps (the passes of ranks fill disjoint columns)
   const int64_t dz = (int64_t)npasses((int)p.W, bwd_rc(p)) * a.ncg * a.BT * a.R * 4;
   w.dz_off = 0;
   w.du_off = (dz + 255) / 256 * 256;
-  w.zp_off = (w.du_off + (int64_t)a.npair * a.RK * p.W * p.D * 4 + 255) / 256 * 256;
+  w.zp_off = (w.du_off + (int64_t)w.slots * a.RK * p.W * p.D * 4 + 255) / 256 * 256;
   w.dxf_off = (w.zp_off + a.BT * zpad_ranks(p) * 2 + 255) / 256 * 256;
   w.total = w.dxf_off + (bwd_f32dx_room(p) ? a.BT * p.D * 4 : 0);
   return w;
@@ -701,9 +706,7 @@ hipError_t launch_bwd(const LrProblem* p, int G) {
   if (np < 1) return hipErrorInvalidValue;
   const bool f32 = bwd_f32dx(p[0]), dxs = bwd_dx_split(p[0]);
   LrBwdArgs a = make_bwd_args(p[0], kBwdTargetWaves, dxs);
-  const BwdWs w = bwd_ws(p[0], a);
-  a.nblk1 = a.nblk;
-  a.nblk = G * a.nblk1;
+  const BwdWs w = bwd_ws(p[0], dxs);
   a.xld = (int)p[0].xld();
   a.dxld = (int)p[0].dxld();
   a.yhd = (int)p[0].yhd();
@@ -739,45 +742,63 @@ hipError_t launch_bwd(const LrProblem* p, int G) {
     for (int g = 0; g < G; ++g) a.grp[g].dx = (char*)p[g].ws + w.dxf_off;
   }
   a.dxsld = 0;
-  for (int i = 0; i < np; ++i) {
-    // pass i: ranks rofs .. (z from column rofs, U and the dU partial rows from
-    // row rofs, dz partial columns from rofs, static_w in the pass that holds
-    // rank R), taps kofs .. (U, static_w and the dU partial columns from tap
-    // kofs; dz partials in the slot of its pass of taps); the residual in the
-    // first pass only
-    const BwdPass& f = ps[i];
-    LrBwdArgs b = a;
-    b.R = f.R;
-    b.RK = f.RK;
-    b.kofs = f.kofs;
-    b.accdx = i > 0;
-    b.residual = a.residual && i == 0;
-    if (f32 && i == np - 1) {  // the last pass adds to the accumulator and stores dx, rounded once
-      b.dxsld = (int)p[0].dxld();
-      for (int g = 0; g < G; ++g) b.grp[g].dxs = p[g].dx;
+  // the passes over the runs that a.sp0 and a.npair name, dU partials from slot slot0 on
+  auto passes = [&](int64_t slot0) {
+    for (int i = 0; i < np; ++i) {
+      // pass i: ranks rofs .. (z from column rofs, U and the dU partial rows from
+      // row rofs, dz partial columns from rofs, static_w in the pass that holds
+      // rank R), taps kofs .. (U, static_w and the dU partial columns from tap
+      // kofs; dz partials in the slot of its pass of taps); the residual in the
+      // first pass only
+      const BwdPass& f = ps[i];
+      LrBwdArgs b = a;
+      b.R = f.R;
+      b.RK = f.RK;
+      b.kofs = f.kofs;
+      b.accdx = i > 0;
+      b.residual = a.residual && i == 0;
+      if (f32 && i == np - 1) {  // the last pass adds to the accumulator and stores dx, rounded once
+        b.dxsld = (int)p[0].dxld();
+        for (int g = 0; g < G; ++g) b.grp[g].dxs = p[g].dx;
+      }
+      for (int g = 0; g < G; ++g) {
+        b.grp[g].z = static_cast<const T*>(a.grp[g].z) + f.rofs;
+        b.grp[g].U = (const T*)p[g].U + f.rofs * WD + f.kofs * D;
+        b.grp[g].sw = p[g].static_w && f.RK > f.R ? (const void*)((const T*)p[g].static_w + f.kofs * D) : nullptr;
+        b.grp[g].part_dz = a.grp[g].part_dz + f.slot * dz_slot + f.rofs;
+        b.grp[g].part_du = a.grp[g].part_du + slot0 * RKWD + f.rofs * WD + f.kofs * D;
+      }
+      if (auditing()) {
+        audit_bwd_pass(b, f.W, f32);
+        continue;
+      }
+      if (dxs) {  // all passes of ranks of these taps in one launch, from the whole problem's ranks
+        if (f.rofs > 0) continue;
+        b.R = a.R;
+        b.RK = a.RK;
+        b.accdx = 0;
+        b.residual = 0;
+        for (int g = 0; g < G; ++g)
+          b.grp[g].sw = p[g].static_w ? (const void*)((const T*)p[g].static_w + f.kofs * D) : nullptr;
+      }
+      if ((e = dispatch_bwd_kernel<T>(b, f.W, rc, f32, p[0].stream)) != hipSuccess) return e;
     }
-    for (int g = 0; g < G; ++g) {
-      b.grp[g].z = static_cast<const T*>(a.grp[g].z) + f.rofs;
-      b.grp[g].U = (const T*)p[g].U + f.rofs * WD + f.kofs * D;
-      b.grp[g].sw = p[g].static_w && f.RK > f.R ? (const void*)((const T*)p[g].static_w + f.kofs * D) : nullptr;
-      b.grp[g].part_dz = a.grp[g].part_dz + f.slot * dz_slot + f.rofs;
-      b.grp[g].part_du = a.grp[g].part_du + f.rofs * WD + f.kofs * D;
-    }
-    if (auditing()) {
-      audit_bwd_pass(b, f.W, f32);
-      continue;
-    }
-    if (dxs) {  // all passes of ranks of these taps in one launch, from the whole problem's ranks
-      if (f.rofs > 0) continue;
-      b.R = a.R;
-      b.RK = a.RK;
-      b.accdx = 0;
-      b.residual = 0;
-      for (int g = 0; g < G; ++g)
-        b.grp[g].sw = p[g].static_w ? (const void*)((const T*)p[g].static_w + f.kofs * D) : nullptr;
-    }
-    if ((e = dispatch_bwd_kernel<T>(b, f.W, rc, f32, p[0].stream)) != hipSuccess) return e;
+    return hipSuccess;
+  };
+  DuParts t(a.nseg, w.slots);
+  for (;; t.next()) {
+    a.sp0 = t.run0;
+    a.npair = t.n;
+    a.nblk1 = a.npair * a.ncg * a.nrp;
+    a.nblk = G * a.nblk1;
+    if (auditing()) audit_range(w.du_off + t.used() * RKWD * 4, w.zp_off);
+    if ((e = passes(t.slot0)) != hipSuccess) return e;
+    if (!t.more()) break;
+    PartialReduce folds[kMaxGroups];
+    for (int g = 0; g < G; ++g) folds[g] = {a.grp[g].part_du, RKWD, t.used(), RKWD, a.grp[g].part_du};
+    if ((e = reduce_partials_multi(folds, G, kFP32, p[0].stream)) != hipSuccess) return e;
   }
+  if (auditing()) audit_range(w.total, p[0].ws_bytes);
   if (dxs) {
     const void* zs[kMaxGroups];
     for (int g = 0; g < G; ++g) zs[g] = a.grp[g].z;
@@ -800,8 +821,8 @@ hipError_t launch_bwd(const LrProblem* p, int G) {
   for (int g = 0; g < G; ++g) {
     const float* pdz = a.grp[g].part_dz;
     const float* pdu = a.grp[g].part_du;
-    jobs[nj++] = {pdu, RKWD, a.npair, R * WD, p[g].dU};
-    jobs[nj++] = {pdu + R * WD, RKWD, a.npair, p[g].static_w ? WD : 0, p[g].dstatic_w};
+    jobs[nj++] = {pdu, RKWD, t.used(), R * WD, p[g].dU};
+    jobs[nj++] = {pdu + R * WD, RKWD, t.used(), p[g].static_w ? WD : 0, p[g].dstatic_w};
     jobs[nj++] = {pdz, a.BT * R, nslot * a.ncg, a.BT * R, p[g].dz};
   }
   return reduce_partials_multi(jobs, nj, p[0].dtype, p[0].stream);
@@ -811,8 +832,8 @@ hipError_t launch_bwd(const LrProblem* p, int G) {
 
 int64_t lr_mfma_ws_bytes(const LrProblem& p) {
   // the plan depends on dy's layout (bwd_dx_split), which the size queries do not see: room for either
-  const int64_t one = bwd_ws(p, make_bwd_args(p, kBwdTargetWaves, false)).total;
-  const int64_t split = bwd_dx_split(p) ? bwd_ws(p, make_bwd_args(p, kBwdTargetWaves, true)).total : 0;
+  const int64_t one = bwd_ws(p, false).total;
+  const int64_t split = bwd_dx_split(contiguous_problem(p)) ? bwd_ws(p, true).total : 0;
   return one > split ? one : split;
 }
 

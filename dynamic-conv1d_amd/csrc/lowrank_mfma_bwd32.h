@@ -114,7 +114,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // passes of ranks without dx (NODX) share one launch: neighbouring blocks take
   // the same rows and channels, so the second pass reads x and dy from the L2
   const int ps = NODX ? lb % a.nrp : 0, cl0 = NODX ? lb / a.nrp : lb;
-  const int cg = cl0 % a.ncg, sp = cl0 / a.ncg;
+  const int cg = cl0 % a.ncg, du_slot = cl0 / a.ncg, sp = a.sp0 + du_slot;
   const int D = a.D, Tn = a.Tn;
   const int d0 = (cg * NW + wave) * 32;
   const int col = d0 + 2 * n;
@@ -573,7 +573,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // ---- dU partial of this run: rows r < RK of U_eff, the wavefront's 32 columns
   // per tap (rows >= RK fall outside the resource; see lowrank_mfma_bwd.hip)
   const int UL = a.uld;
-  const rsrc_t rdu = make_rsrc(part_du + (int64_t)sp * a.dupr * UL, lr_dupart_bytes(RK, UL, a.kofs, D));
+  const rsrc_t rdu = make_rsrc(part_du + (int64_t)du_slot * a.dupr * UL, lr_dupart_bytes(RK, UL, a.kofs, D));
   const int du_lane = chv ? (4 * q * UL + col) * 4 : kOobLane;
 #pragma unroll
   for (int k = 0; k < W; ++k)

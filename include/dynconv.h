@@ -179,7 +179,8 @@ int dc_lowrank_path(int64_t B, int64_t T, int64_t D, int64_t R, int64_t W, int d
  * the backward) the dU partial; per tensor the range of the longest run.
  * Writes up to max_pairs pairs (bytes, bound) to out, where each count must
  * lie in [0, bound] for every out-of-range offset the kernel uses to stay out
- * of range, and returns the number of pairs (0 for the generic kernels), or a
+ * of range, and (in the backward) the ends of the workspace's parts with the
+ * bytes there are, and returns the number of pairs (0 for the generic kernels), or a
  * negative dc_status.  Launches nothing and makes no HIP call. */
 int64_t dc_lowrank_plan_ranges(int64_t B, int64_t T, int64_t D, int64_t R, int64_t W, int dtype, int has_static,
                                int bwd, int64_t* out, int64_t max_pairs);
@@ -230,7 +231,9 @@ int64_t dc_lowrank_bwd_grouped_ws_bytes(int64_t G, int64_t B, int64_t T, int64_t
  * when dy_hd = 0 and head-major [B, D/dy_hd, T, dy_hd] otherwise (the layout
  * of dc_lowrank_fwd_grouped's y_hd).  dstatic_w is NULL exactly when static_w
  * is.  Per group, results are bitwise those of dc_lowrank_bwd (with a head
- * dim: when it is a multiple of 64, else the generic kernels).  Replaces
+ * dim: when it is a multiple of 64, else the generic kernels; dU and dstatic_w
+ * to their sums' last bits where rows of x or dx are so far apart that a run of
+ * rows has to be shorter than the contiguous call's).  Replaces
  * README.md:57-110's three backwards (lowrank.py:251-299 each) and the
  * concatenation of dq, dk, dv.  z_eff is NULL or the array of G buffers (of
  * z_eff_bytes each) that dc_lowrank_fwd_grouped filled. */
