@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
 #pragma unroll
     for (int m = 0; m < NR; ++m) in.xr[m] = bload64(rx, xlane_off + xtoff + (m - (W - 1)) * xrowb);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) in.dyr[m] = bload64<kNt>(rdy, lane_off + toff + m * rowb);
+    for (int m = 0; m < 4; ++m) in.dyr[m] = bload64(rdy, lane_off + toff + m * rowb);  // nontemporal: 71 us for 62 (R63 + static)
     in.zr.load(rz, ylive ? (tile * 16 + n - rb) * zld * 2 : kOobTile, zr, q);
   };
   // Tap k's weights of the lane's rows for channel 4n+j, accumulator started at w0.
