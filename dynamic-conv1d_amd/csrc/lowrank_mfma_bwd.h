@@ -72,9 +72,10 @@ template <typename T, bool F32> struct DxVec {
   __device__ static __forceinline__ type load(rsrc_t r, int off) { return bload32(r, off); }
   // 16-bit rows leave in 64-byte pieces (half lines): the default policy lets the
   // L2 join two wavefronts' halves (B2 T8192 D4096 R31 + static backward 129 ->
-  // 125 us against nontemporal stores, W 8 at R15 85 -> 83 us)
+  // 125 us against nontemporal stores, W 8 at R15 85 -> 83 us); NT: lr_bwd_t32's NTP
+  template <bool NT>
   __device__ static __forceinline__ void store(type v, rsrc_t r, int off) {
-    __builtin_amdgcn_raw_buffer_store_b32(v, r, off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(v, r, off, 0, NT ? kNt : 0);
   }
   __device__ static __forceinline__ float get(type v, int j) { return Mma16<T>::to_f(Pair::elem(v, j)); }
   __device__ static __forceinline__ type make(const float* f) { return pack2<T>(f[0], f[1]); }
@@ -83,6 +84,7 @@ template <typename T> struct DxVec<T, true> {
   typedef u32x2 type;
   static constexpr int ES = 4;
   __device__ static __forceinline__ type load(rsrc_t r, int off) { return bload64(r, off); }
+  template <bool NT>
   __device__ static __forceinline__ void store(type v, rsrc_t r, int off) { bstore64<true>(v, r, off); }
   __device__ static __forceinline__ float get(const type& v, int j) { return __uint_as_float(v[j]); }
   __device__ static __forceinline__ type make(const float* f) {

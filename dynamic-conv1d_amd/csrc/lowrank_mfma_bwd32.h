@@ -92,6 +92,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   typedef DxVec<T, DXM == 1 || DXM == 2> DV;
   typedef DxVec<T, DXM == 1> DVS;
   typedef ZRaw<T, RC, true> ZR;
+  // Passes that add to an earlier one's dx (ACC): when its rows are loaded (load_dxo).
+  // Two rank chunks at W 4 and one at any W have no registers for them beside a
+  // tile's fp32 rows, and take them before the last tap; the fp32 accumulator's at W <=
+  // 2 come with the tile, which is too short to hide them, at W 3 at its start.  And the
+  // passes that stream more than the last-level cache keeps (an fp32 accumulator, or
+  // two rank chunks at W 4) read dy and store dx nontemporal.  B4 T4096 D2048, rows
+  // held from the tile's start with the open ones carried (8-12 registers spilled),
+  // and now: R31 + static W 8 153 -> 145 us, W 12 226 -> 213, W 20 513 -> 451, R64 W 20
+  // 1115 -> 946, R127 + static W 8 932 -> 815, R160 W 1 379 -> 367, R255 + static W 4
+  // 916 -> 789.  Rows with the tile at W 4 spill (W 20: 788).
+  enum { kDxoTile, kDxoLastTap, kDxoAhead };
+  constexpr int DXO = RC == 1 || DXM == 0 || W == 4 ? kDxoLastTap : W <= 2 ? kDxoAhead : kDxoTile;
+  constexpr bool NTP = RC == 2 && (DXM == 1 || DXM == 2 || (ACC && W == 4));
   __shared__ u32x4 us[NW][UREG ? 1 : W * RC * 64];
   __shared__ __attribute__((aligned(16))) uint8_t gtile[NW][8 * GPL];
   __shared__ __attribute__((aligned(16))) float dzred[2][DZB][NW][RC * 512];
@@ -153,6 +166,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int xlane_off = chv ? (8 * q * a.xld + col) * 2 : kOobLane;
   const int dxlane_off = chv ? (8 * q * a.dxld + col) * DV::ES : kOobLane;
   const int dxslane_off = chv ? (8 * q * dxsld + col) * DVS::ES : kOobLane;
+  // ACC: the earlier passes' dx of the rows that close_rows(tile) stores
+  auto load_dxo = [&](int tile, typename DV::type(&dxo)[ACC ? 8 : 1]) {
+    if constexpr (ACC) {
+      const int cur = tile < tile1 ? dxlane_off + (tile * 32 - rb - kofs) * dxrowb : kOobTile;
+      const int prev = tile > tile0 ? dxlane_off + ((tile - 1) * 32 - rb - kofs) * dxrowb : kOobTile;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        dxo[i] = DV::load(rdx, (W > 1 && i >= kFirstOpen && q == 3 ? prev : cur) + i * dxrowb);
+    }
+  };
   const int zrow = 8 * (n >> 2) + (n & 3);  // tile row of the lane's z operand in half 0 (half 1: + 4)
 
   // Tile inputs (buffer loads: rows outside the sequence and channels past D
@@ -162,6 +185,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     uint32_t xr[NX], dyr[8];
     ZR zraw[RC == 2 ? 1 : 2];
     u32x4 z32[RC == 2 ? 2 : 1];
+    typename DV::type dxo[ACC && DXO == kDxoAhead ? 8 : 1];
   };
   TileIn in[NBUF];
   auto load_tile = [&](TileIn& in, int tile) {
@@ -171,7 +195,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int m = 0; m < NX; ++m) in.xr[m] = LV::load(rx, xlane_off + xtoff + (m + 8 - NX) * xrowb);
 #pragma unroll
-    for (int m = 0; m < 8; ++m) in.dyr[m] = LV::load(rdy, lane_off + toff + m * rowb);
+    for (int m = 0; m < 8; ++m) in.dyr[m] = bload32<NTP ? kNt : 0>(rdy, lane_off + toff + m * rowb);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int zoff = ylive ? (tile * 32 + zrow + 4 * h - rb) * zld * 2 : kOobTile;
@@ -180,6 +204,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       else
         in.zraw[h].load(rz, zoff, zr, q);
     }
+    if constexpr (ACC && DXO == kDxoAhead) load_dxo(tile, in.dxo);
   };
 #pragma unroll
   for (int i = 0; i < NBUF; ++i) load_tile(in[i], tile0 + i);
@@ -359,7 +384,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   float carry[NO][2];
 #pragma unroll
   for (int i = 0; i < NO; ++i) carry[i][0] = carry[i][1] = 0.f;
-  typename DV::type dxo_carry[ACC ? NO : 1] = {};
   auto close_rows = [&](const float(&own)[8][2], const float(&S)[NO][2], int tile,
                         const typename DV::type(&dxo)[ACC ? 8 : 1]) {
     const int src = ((lane + 16) & 63) << 2;  // ds_bpermute byte index of the group below
@@ -384,18 +408,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       }
       if constexpr (ACC) {  // a later pass adds to the stored rows
         typename DV::type o = dxo[i];
-        if (open) o = top ? dxo_carry[i - kFirstOpen] : o;
 #pragma unroll
         for (int j = 0; j < 2; ++j) v[j] += DV::get(o, j);
       }
-      DVS::store(DVS::make(v), rdxs, (open ? open_off : cur_off) + i * dxsrowb);
+      DVS::template store<NTP>(DVS::make(v), rdxs, (open ? open_off : cur_off) + i * dxsrowb);
     }
     if constexpr (W > 1) {
 #pragma unroll
       for (int i = 0; i < NO; ++i) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) carry[i][j] = own[kFirstOpen + i][j];
-        if constexpr (ACC) dxo_carry[i] = dxo[kFirstOpen + i];
       }
     }
   };
@@ -425,9 +447,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     ZA zA[2] = {z_op(in, tile, 0), z_op(in, tile, 1)};
     __builtin_amdgcn_sched_barrier(0);
     typename DV::type dxo[ACC ? 8 : 1] = {};
-    if constexpr (ACC) {  // the earlier passes' dx of the tile's rows
+    if constexpr (ACC && DXO == kDxoTile) load_dxo(tile, dxo);
+    if constexpr (ACC && DXO == kDxoAhead) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) dxo[i] = DV::load(rdx, dxlane_off + (tile * 32 - rb - kofs + i) * dxrowb);
+      for (int i = 0; i < 8; ++i) dxo[i] = in.dxo[DXO == kDxoAhead ? i : 0];
     }
     load_tile(in, tile + NBUF);
     __builtin_amdgcn_sched_barrier(0);  // the next tile's loads go out before this tile's products
@@ -459,6 +482,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 #pragma unroll
     for (int k = 0; k < W; ++k) {
+      if (ACC && DXO == kDxoLastTap && k == W - 1) {
+        load_dxo(tile, dxo);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       // G_k of the lane's rows and channels (fp32 products, rounded once); the
       // wave barriers keep the compiler from moving an LDS write above another
       // lane's read (the hardware keeps a wavefront's LDS order)
@@ -566,8 +593,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int j = 0; j < 2; ++j) scatter(tap_w(za, tap_op(k, j), 0.f), dyf, k, j, h, own, S);
     }
-    const typename DV::type none[ACC ? 8 : 1] = {};
-    close_rows(own, S, tile1, none);
+    typename DV::type dxo[ACC ? 8 : 1] = {};
+    load_dxo(tile1, dxo);
+    close_rows(own, S, tile1, dxo);
   }
 
   // ---- dU partial of this run: rows r < RK of U_eff, the wavefront's 32 columns
