@@ -1,7 +1,7 @@
 // Shared pieces of the lowrank backward on gfx950 matrix cores (bf16 / fp16):
 // the launch arguments and the row-piece types of its two kernels, lr_bwd_t32
-// (lowrank_mfma_bwd32.h: one and two rank chunks) and lr_bwd_mfma
-// (lowrank_mfma_bwd.hip: three and four), and the host's launch of the first.
+// (lowrank_mfma_bwd32.h) and lr_bwd_mfma (lowrank_mfma_bwd.hip), and the host's
+// launch of the first.
 #pragma once
 
 #include "lowrank_mfma.h"
@@ -22,12 +22,12 @@ struct LrBwdGroup {
 
 struct LrBwdArgs {
   int Tn, D, R, RK, residual;
-  int nch;    // channel chunks of one wavefront (32 channels, or 64 in lr_bwd_mfma)
+  int nch;    // channel chunks of one wavefront (32 or 64 channels)
   int ncg;    // chunk groups of 256 channels: one workgroup column
   int seg;    // tiles per run
   int nspb;   // runs per sequence
   int nseg;   // B * nspb
-  int npair;  // workgroup rows of a launch: one run, one dU partial each (nseg, or a part of the runs: DuParts)
+  int npair;  // workgroup rows of a launch: a run, a dU partial each (lr_bwd_mfma: one or two; nseg, or a part: DuParts)
   int sp0;    // first run of the launch; its dU partial is part_du's first
   int nblk;   // ncg * npair * nrp * groups
   int nblk1;  // blocks per group

@@ -7,29 +7,33 @@ namespace dc {
 //
 // Host side of the backward (launch plans, passes, workspace), and the kernel of
 // the one-pass problems of three and four rank chunks (kernel ranks 33-48 at
-// W <= 2, 49-64 at W 1).  One and two rank chunks, and every problem that runs
-// as passes of ranks, take lr_bwd_t32 (lowrank_mfma_bwd32.h).
+// W <= 2, 49-64 at W 1) and of those of one and two chunks that stream past the
+// last-level cache (bwd_streams).  Other problems of one and two chunks, and every
+// problem that runs as passes, take lr_bwd_t32 (lowrank_mfma_bwd32.h).
 //
 // lr_bwd_mfma: one pass over x and dy produces dx, dz, dU and dstatic_w
 // (reference: lowrank.py:87-140 and 159-205, two kernels that both read dy).
-// A wavefront owns 16 rows x 64 channels; lane l = 16q + n owns rows 4q..4q+3
-// and the channels 4n..4n+3 (one 8-byte load per row).  With
+// A wavefront owns 16 rows x CPW channels (64, or 32 at two rank chunks); lane
+// l = 16q + n owns rows 4q..4q+3 and the NJ = CPW/16 channels NJ*n .. (one 8- or
+// 4-byte load per row).  With
 // G_k[t, d] = bf16(dy[t, d] * x[t-k, d]) (the reference also rounds this
 // product to bf16 before its dot products, lowrank.py:128):
 //   * dU[r, kD+d] += sum_t z_eff[t, r] G_k[t, d]: MFMA with K = the 16 rows; the
-//     lane's four G values of column 4n+j are the B operand.
+//     lane's four G values of column NJ*n+j are the B operand.
 //   * dz[t, r] += sum_d G_k[t, d] U_eff[r, kD+d]: K = 32 channels; the packed dU
 //     operands go through the wavefront's LDS slot and come back by row with
 //     transposing reads (ds_read_b64_tr_b16).
 //   * Tap weights Kw[t, k, :] = z_eff[t, :] U_eff[:, k]: one 16x16x16 MFMA per
-//     rank chunk.  The residual's dy rides on tap 0: its accumulator starts at 1.
+//     rank chunk, or one 16x16x32 over two.  The residual's dy rides on tap 0:
+//     its accumulator starts at 1.
 //   * dx[t, d] = sum_k dy[t+k, d] Kw[t+k, k, d] (+ dy) in scatter form: dy[s]
-//     Kw[s, k] goes to row s-k; the sums for the group above (W 2) pass up with
-//     a ds_bpermute, and group 3's open row waits one tile.
-// A workgroup is four wavefronts on 256 adjacent channels of one run of rows.
-// dz sums over the 256 channels are added in LDS in wave order, dU accumulates
-// in registers over the run; both go out as fp32 partials that reduce_partials
-// sums in a fixed order.
+//     Kw[s, k] goes to row s-k; the sums for the group above pass up with a
+//     ds_bpermute each, and group 3's open rows wait one tile.
+// A workgroup covers 256 adjacent channels of one run of rows, or of two (one
+// rank chunk: half the dU partials).  dz sums over the 256 channels are added in
+// LDS in wave order, dU accumulates in registers over the run (the second run's
+// is added to the first's at the end); both go out as fp32 partials that
+// reduce_partials sums in a fixed order.
 //
 // Passes of taps (lr_bwd_t32): a launch holds the operands and accumulators of
 // at most pass_taps(W, RC) taps, so wider problems run as consecutive launches
@@ -43,24 +47,52 @@ namespace dc {
 // q / k / v convolutions read x out of a fused [B, T, 3D] projection and write
 // dx into its gradient.
 
-// U_eff operands of one wavefront's 64-channel chunk, staged once per run: the
+// NJ (4 or 2) 16-bit channels of one row held by a lane: one 8- or 4-byte unit.
+template <int NJ> struct LaneVec;
+template <> struct LaneVec<4> {
+  typedef u32x2 type;
+  template <int AUX>
+  __device__ static __forceinline__ type load(rsrc_t r, int off) { return bload64<AUX>(r, off); }
+  __device__ static __forceinline__ void store(type v, rsrc_t r, int off) { bstore64<true>(v, r, off); }
+  __device__ static __forceinline__ uint32_t elem(const type& v, int j) { return elem16x2(v, j); }
+  template <typename T>
+  __device__ static __forceinline__ type pack(const float* f) {
+    return type{pack2<T>(f[0], f[1]), pack2<T>(f[2], f[3])};
+  }
+};
+template <> struct LaneVec<2> {
+  typedef uint32_t type;
+  template <int AUX>
+  __device__ static __forceinline__ type load(rsrc_t r, int off) { return bload32<AUX>(r, off); }
+  __device__ static __forceinline__ void store(type v, rsrc_t r, int off) {
+    __builtin_amdgcn_raw_buffer_store_b32(v, r, off, 0, kNt);
+  }
+  __device__ static __forceinline__ uint32_t elem(const type& v, int j) { return j ? (v >> 16) : (v & 0xFFFFu); }
+  template <typename T>
+  __device__ static __forceinline__ type pack(const float* f) {
+    return pack2<T>(f[0], f[1]);
+  }
+};
+
+// U_eff operands of one wavefront's channels, staged once per run: the
 // tap-weight operands in registers, the dz operands in LDS.  For tap k and rank
 // chunk c, lane (q, n) holds
-//   uw[j] (j < 4): ranks 16c+4q..16c+4q+3 of channel 4n+j, packed (B operand of
-//                  the 16x16x16 tap-weight MFMA);
-//   uz[s] (s < 2): rank 16c+n, channels 32s+8q..32s+8q+7 as they lie in U (B
+//   uw[j] (j < NJ): ranks 16c+4q..16c+4q+3 of channel NJ*n+j, packed (B operand
+//                  of the 16x16x16 tap-weight MFMA); not with two chunks (stage_uw32);
+//   uz[s] (s < NS): rank 16c+n, channels 32s+8q..32s+8q+7 as they lie in U (B
 //                  operand of the 16x16x32 dz MFMA).
-template <int W, int RC>
-__device__ __forceinline__ void stage_uops(u32x2 (&uw)[W * RC * 4], u32x4* __restrict__ uz_lds,
+template <int W, int RC, int NJ, int NS, bool STAGE_UW>
+__device__ __forceinline__ void stage_uops(u32x2 (&uw)[STAGE_UW ? W * RC * NJ : 1], u32x4* __restrict__ uz_lds,
                                            const uint16_t* __restrict__ U, const uint16_t* __restrict__ sw, int R,
                                            int RK, int D, int uld, int d0, int q, int n, int lane) {
+  typedef LaneVec<NJ> LV;
   // Buffer loads, all issued before the first use: rows r >= R of U and lanes
   // outside D read 0; the static row (r == R < RK) is read from sw and OR-ed in.
   const rsrc_t ru = make_rsrc(U, lr_u_bytes(R, uld, 0, D, 2));
   const rsrc_t rs = make_rsrc(sw, lr_sw_bytes(RK > R, W, D, 2));
-  const int cw = d0 + 4 * n < D ? (d0 + 4 * n) * 2 : kOobLane;  // the lane's tap-weight channels
-  u32x2 rows[W][RC][4];
-  u32x4 zr[W][RC][2];
+  const int cw = d0 + NJ * n < D ? (d0 + NJ * n) * 2 : kOobLane;  // the lane's tap-weight channels
+  typename LV::type rows[W][RC][4];
+  u32x4 zr[W][RC][NS];
 #pragma unroll
   for (int k = 0; k < W; ++k)
 #pragma unroll
@@ -69,12 +101,13 @@ __device__ __forceinline__ void stage_uops(u32x2 (&uw)[W * RC * 4], u32x4* __res
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) {
         const int r = 16 * c + 4 * q + kk;
-        rows[k][c][kk] = bload64(ru, r < R ? cw + (r * uld + k * D) * 2 : kOobLane) |
-                         bload64(rs, has_static && r == R ? cw + k * D * 2 : kOobLane);
+        if constexpr (STAGE_UW)
+          rows[k][c][kk] = LV::template load<0>(ru, r < R ? cw + (r * uld + k * D) * 2 : kOobLane) |
+                           LV::template load<0>(rs, has_static && r == R ? cw + k * D * 2 : kOobLane);
       }
       const int r = 16 * c + n;
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
+      for (int s2 = 0; s2 < NS; ++s2) {
         const int dd = d0 + 32 * s2 + 8 * q;  // multiple of 8; D % 8 == 0, so dd < D means dd + 8 <= D
         const int cz = dd < D ? dd * 2 : kOobLane;
         zr[k][c][s2] = bload128(ru, r < R ? cz + (r * uld + k * D) * 2 : kOobLane) |
@@ -86,33 +119,85 @@ __device__ __forceinline__ void stage_uops(u32x2 (&uw)[W * RC * 4], u32x4* __res
 #pragma unroll
     for (int c = 0; c < RC; ++c) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const u32x2(&rw)[4] = rows[k][c];
-        uw[(k * RC + c) * 4 + j][0] = elem16x2(rw[0], j) | (elem16x2(rw[1], j) << 16);
-        uw[(k * RC + c) * 4 + j][1] = elem16x2(rw[2], j) | (elem16x2(rw[3], j) << 16);
+      for (int j = 0; j < (STAGE_UW ? NJ : 0); ++j) {
+        const typename LV::type(&rw)[4] = rows[k][c];
+        uw[(k * RC + c) * NJ + j][0] = LV::elem(rw[0], j) | (LV::elem(rw[1], j) << 16);
+        uw[(k * RC + c) * NJ + j][1] = LV::elem(rw[2], j) | (LV::elem(rw[3], j) << 16);
       }
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) uz_lds[((k * RC + c) * 2 + s2) * 64 + lane] = zr[k][c][s2];
+      for (int s2 = 0; s2 < NS; ++s2) uz_lds[((k * RC + c) * NS + s2) * 64 + lane] = zr[k][c][s2];
     }
 }
 
-template <typename T, int W, int RC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) void lr_bwd_mfma(LrBwdArgs a) {
-  static_assert(W <= 2 && (RC == 3 || RC == 4), "the one-pass shapes of three and four rank chunks");
-  typedef ZRaw<T, RC, true> ZR;   // 8-byte z loads: rows of zld % 4 == 0 elements
-  constexpr int NR = W + 3;       // x rows 4q-W+1 .. 4q+3 per lane
+// Tap-weight operands for K = 32 ranks (two rank chunks): lane (q, n) gives
+// ranks 8q..8q+7 of channel NJ*n+j, packed (B operand of the 16x16x32 MFMA
+// whose A is z_eff row n, ranks 8q..8q+7).  Row R (< RK) is static_w.
+template <int W, int NJ>
+__device__ __forceinline__ void stage_uw32(u32x4 (&uw)[W * NJ], const uint16_t* __restrict__ U,
+                                           const uint16_t* __restrict__ sw, int R, int RK, int D, int uld, int d0,
+                                           int q, int n) {
+  typedef LaneVec<NJ> LV;
+  const rsrc_t ru = make_rsrc(U, lr_u_bytes(R, uld, 0, D, 2));
+  const rsrc_t rs = make_rsrc(sw, lr_sw_bytes(RK > R, W, D, 2));
+  const int cw = d0 + NJ * n < D ? (d0 + NJ * n) * 2 : kOobLane;
+  typename LV::type rows[W][8];
+#pragma unroll
+  for (int k = 0; k < W; ++k)
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+      const int r = 8 * q + kk;
+      rows[k][kk] = LV::template load<0>(ru, r < R ? cw + (r * uld + k * D) * 2 : kOobLane) |
+                    LV::template load<0>(rs, RK > R && r == R ? cw + k * D * 2 : kOobLane);
+    }
+#pragma unroll
+  for (int k = 0; k < W; ++k)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      u32x4 v;
+#pragma unroll
+      for (int h = 0; h < 4; ++h) v[h] = LV::elem(rows[k][2 * h], j) | (LV::elem(rows[k][2 * h + 1], j) << 16);
+      uw[k * NJ + j] = v;
+    }
+}
+
+// A operands of the tap-weight MFMA: four ranks per rank chunk (16x16x16) or,
+// with two rank chunks, eight ranks (16x16x32).
+template <int RC> struct ZOp { u32x2 c[RC]; };
+template <> struct ZOp<2> { u32x4 v; };
+
+// CPW channels to a wavefront, NRW runs to a workgroup (bwd_shape).
+template <typename T, int W, int RC, int NRW, int CPW>
+__global__ __launch_bounds__(64 * (256 / CPW) * NRW)
+__attribute__((amdgpu_waves_per_eu(RC <= 2 ? 2 : 1, 8))) void lr_bwd_mfma(LrBwdArgs a) {
+  static_assert(W <= 4 && W * RC <= 8, "tap-weight operands in registers");
+  static_assert(NRW == 1 || (RC == 1 && CPW == 64), "two runs per workgroup: one rank chunk");
+  constexpr int NJ = CPW / 16;     // channels per lane
+  constexpr int NS = CPW / 32;     // 32-channel K blocks of the dz MFMA
+  constexpr int NCW = 256 / CPW;   // channel-chunk wavefronts per run: 256 channels per workgroup
+  constexpr int NW = NCW * NRW;    // wavefronts per workgroup
+  constexpr bool K32 = RC == 2;    // tap weights over 32 ranks in one 16x16x32 MFMA (z rows of exactly 32 ranks)
+  constexpr int NR = W + 3;        // x rows 4q-W+1 .. 4q+3 per lane
+  constexpr int NSC = W > 1 ? W - 1 : 1;  // open rows of a group (none at W 1)
+  constexpr int kFirstOpen = 5 - W;       // rows kFirstOpen .. 3 take the group below's sums
+  typedef LaneVec<NJ> LV;
+  typedef ZOp<RC> ZO;
+  typedef ZRaw<T, RC, true> ZR;  // 8-byte z loads: rows of zld % 4 == 0 elements
+  constexpr int NUZ = W * RC * NS;  // dz operands per lane
   // G tile in LDS, transposed: channel c's rows 4p..4p+3 (8 bytes) at byte
   // p*GPL + 8c + 8(c/16).  The pad of 8 bytes per 16 channels keeps both access
   // patterns within two-way bank conflicts.
-  constexpr int GPL = 8 * 64 + 32;  // bytes per 4-row plane
-  __shared__ u32x4 uz_lds[4][W * RC * 2 * 64];
-  __shared__ __attribute__((aligned(16))) uint8_t gtile[4][4 * GPL];
-  // dz sums of the workgroup's chunks (double-buffered: one barrier per tile).
-  // Row r, rank n of a tile sits at (16r + n) ^ ((r / 4) << 4): the XOR puts the
-  // four row groups a lane quarter writes at once in different banks.
-  __shared__ float dzred[2][4][RC * 256];
+  constexpr int GPL = 8 * CPW + CPW / 2;  // bytes per 4-row plane
+  __shared__ u32x4 uz_lds[NW][NUZ * 64];
+  __shared__ __attribute__((aligned(16))) uint8_t gtile[NW][4 * GPL];
+  // dz sums of the workgroup's chunks, gathered for DZB tiles (double-buffered:
+  // one barrier per batch).  Row r, rank n of a tile sits at (16r + n) ^ ((r /
+  // 4) << 4): the XOR puts the four row groups a lane quarter writes at once in
+  // different banks.
+  constexpr int DZB = RC == 1 ? 4 : RC == 2 && W >= 2 ? 2 : 1;
+  __shared__ float dzred[2][NRW][NCW][DZB][RC * 256];
 
   const int lane = threadIdx.x & 63, wave = wave_id();
+  const int cw = wave % NCW, rw = wave / NCW;  // chunk and run of this wavefront in the workgroup
   const int q = lane >> 4, n = lane & 15;
   const int lb0 = xcd_remap(blockIdx.x, a.nblk);
   const int g = __builtin_amdgcn_readfirstlane(lb0 / a.nblk1);
@@ -126,25 +211,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
   uint16_t* __restrict__ dx = reinterpret_cast<uint16_t*>(gp->dx);
   float* __restrict__ part_dz = gp->part_dz;
   float* __restrict__ part_du = gp->part_du;
-  const int cg = lb % a.ncg, du_slot = lb / a.ncg, sp = a.sp0 + du_slot;
+  const int cg = lb % a.ncg, du_slot = lb / a.ncg, sp = a.sp0 + du_slot * NRW;
   const int D = a.D, Tn = a.Tn;
-  const int d0 = (cg * 4 + wave) * 64;
-  const int col = d0 + 4 * n;
-  const bool chv = col < D;  // the lane's 4 channels inside D (D % 8 == 0: all or none)
+  const int d0 = (cg * NCW + cw) * CPW;
+  const int col = d0 + NJ * n;
+  const bool chv = col < D;  // the lane's NJ channels inside D (D % 8 == 0: all or none)
   const int ntile = (Tn + 15) >> 4;
-  // the workgroup's run: tiles [tile0, tile1) of sequence b, whose buffer resources start at row rb
-  const int b = sp / a.nspb;
-  const int tile0 = (sp - b * a.nspb) * a.seg;
-  const int tile1 = min(tile0 + a.seg, ntile);
-  const int rb = run_base_row(tile0);
-  const int64_t row0 = (int64_t)b * Tn, rrow = row0 + rb;
+  // Run s: tiles [tile0, tile1) of sequence b, whose buffer resources start at
+  // row rb.  A workgroup's last run can lie past nseg (odd nseg): it has no tiles.
+  struct Run {
+    int tile0, tile1, rb;
+    int64_t row0;
+  };
+  auto run_of = [&](int s) {
+    Run r{0, 0, 0, 0};
+    if (s < a.nseg) {
+      const int b = s / a.nspb;
+      r.tile0 = (s - b * a.nspb) * a.seg;
+      r.tile1 = min(r.tile0 + a.seg, ntile);
+      r.rb = run_base_row(r.tile0);
+      r.row0 = (int64_t)b * Tn;
+    }
+    return r;
+  };
+  Run runs[NRW];
+  int nit = 0;  // iterations of every wavefront: the longest run of the workgroup
+#pragma unroll
+  for (int i = 0; i < NRW; ++i) {
+    runs[i] = run_of(sp + i);
+    nit = max(nit, runs[i].tile1 - runs[i].tile0);
+  }
+  const Run me = rw == 0 ? runs[0] : runs[NRW - 1];
+  const int tile0 = me.tile0, tile1 = me.tile1, rb = me.rb;
+  const int64_t row0 = me.row0, rrow = row0 + rb;
   const int R = a.R, RK = a.RK;
   u32x4* __restrict__ my_uz = uz_lds[wave];
-  // G^T write position of the lane's channel 4n (plus 8j), and the transposed-read
+  // G^T write position of the lane's channel NJ*n (plus 8j), and the transposed-read
   // position that returns row n, channels 8q..8q+3 (plus 32 for 8q+4..8q+7, plus
   // 8*32+16 per 32-channel block)
   uint8_t* const my_g = gtile[wave];
-  const int gw_lane = q * GPL + 32 * n + (n / 4) * 8;
+  const int gw_lane = q * GPL + NJ * 8 * n + (n / (16 / NJ)) * 8;
   const int gr_lane = (n & 3) * GPL + (8 * q + (n >> 2)) * 8 + (q >> 1) * 8;
   const float res = a.residual ? 1.f : 0.f;  // tap 0's weight + 1: the residual term dy
   // dy is [B, T, D] (yhd == D) or head-major [B, D/yhd, T, yhd] (yhd % 64 == 0: a
@@ -156,14 +262,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
   const rsrc_t rdx = run_rsrc(dx + rrow * a.dxld, Tn - rb, dxrowb);
   const int zld = a.zld, zr = a.zr, zrk = a.zrk;
   const rsrc_t rz = run_rsrc(z + rrow * zld, Tn - rb, zld * 2);
-  const rsrc_t rpz = run_rsrc(part_dz + ((int64_t)cg * a.BT + rrow) * a.dzld, Tn - rb, a.dzld * 4);
   // byte offsets of the lane's row-4q channels in dy, x and dx
   const int lane_off = chv ? (4 * q * yhd + col - head * yhd) * 2 : kOobLane;
   const int xlane_off = chv ? (4 * q * a.xld + col) * 2 : kOobLane;
   const int dxlane_off = chv ? (4 * q * a.dxld + col) * 2 : kOobLane;
 
-  // Identity as the B operand: lane (q, n) gives rows 4q..4q+3 of column n.
+  u32x2 uw[K32 ? 1 : W * RC * NJ];  // staged below, after the first tile's loads are issued
+  u32x4 uw32[K32 ? W * NJ : 1];
+  // Identity (or, for 32 ranks, rank-selection) matrices as the B operand that transposes z_eff.
   u32x2 ident;
+  u32x4 sel[K32 ? 2 : 1];
   {
     const uint32_t one = Mma16<T>::kOne;
     uint32_t e[4];
@@ -171,90 +279,139 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
     for (int kk = 0; kk < 4; ++kk) e[kk] = (4 * q + kk == n) ? one : 0u;
     ident[0] = e[0] | (e[1] << 16);
     ident[1] = e[2] | (e[3] << 16);
+    if constexpr (K32) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {
+          const uint32_t lo = (8 * q + 2 * h == 16 * c + n) ? one : 0u;
+          const uint32_t hi = (8 * q + 2 * h + 1 == 16 * c + n) ? one : 0u;
+          sel[c][h] = lo | (hi << 16);
+        }
+    }
   }
-  u32x2 uw[W * RC * 4];
-  f32x4 du[W][RC][4];
+  f32x4 du[W][RC][NJ];
 #pragma unroll
   for (int k = 0; k < W; ++k)
 #pragma unroll
     for (int c = 0; c < RC; ++c)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) du[k][c][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NJ; ++j) du[k][c][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // Tile inputs (buffer loads: out-of-range rows / channels read as 0).  Two
   // buffers alternate: while one tile is computed the next one's loads are in
   // flight.  A tile past the run reads the out-of-range offset kOobTile; dy and z
-  // of the tile after the run are read too (its first row closes the last dx row).
+  // of the tile after the run are read too (its first rows close the last dx rows).
+  // dy rows are read once: nontemporal (B4 T4096 D2048 R16 60.0 -> 58.8 us), but
+  // not in the short tiles of W 1 and the long ones of three and four chunks, which
+  // wait for them (R63 + static W 1 71 -> 62 us without).
   struct TileIn {
-    u32x2 xr[NR], dyr[4];
+    typename LV::type xr[NR], dyr[4];
     ZR zr;
+    u32x4 z32;
   };
   auto load_tile = [&](int tile, TileIn& in) {
-    const bool live = tile < tile1, ylive = tile <= tile1;
+    const bool live = tile < tile1, ylive = W > 1 ? tile <= tile1 : live;
     const int xtoff = live ? (tile * 16 - rb) * xrowb : kOobTile;
     const int toff = ylive ? (tile * 16 - rb) * rowb : kOobTile;
 #pragma unroll
-    for (int m = 0; m < NR; ++m) in.xr[m] = bload64(rx, xlane_off + xtoff + (m - (W - 1)) * xrowb);
+    for (int m = 0; m < NR; ++m) in.xr[m] = LV::template load<0>(rx, xlane_off + xtoff + (m - (W - 1)) * xrowb);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) in.dyr[m] = bload64(rdy, lane_off + toff + m * rowb);  // nontemporal: 71 us for 62 (R63 + static)
-    in.zr.load(rz, ylive ? (tile * 16 + n - rb) * zld * 2 : kOobTile, zr, q);
+    for (int m = 0; m < 4; ++m) in.dyr[m] = LV::template load<W == 1 || RC >= 3 ? 0 : kNt>(rdy, lane_off + toff + m * rowb);
+    if constexpr (K32)
+      in.z32 = bload128(rz, ylive ? ((tile * 16 + n - rb) * zld + 8 * q) * 2 : kOobTile);
+    else
+      in.zr.load(rz, ylive ? (tile * 16 + n - rb) * zld * 2 : kOobTile, zr, q);
   };
-  // Tap k's weights of the lane's rows for channel 4n+j, accumulator started at w0.
-  auto tap_w = [&](const u32x2(&za)[RC], int k, int j, float w0) {
+  auto z_op = [&](const TileIn& in, int tile) {
+    ZO o;
+    if constexpr (K32)
+      o.v = in.z32;
+    else
+      in.zr.finish(o.c, tile * 16 + n, zr, zrk, Tn, q);
+    return o;
+  };
+  // Tap k's weights of the lane's rows for channel NJ*n+j, accumulator started at w0.
+  auto tap_w = [&](const ZO& za, int k, int j, float w0) {
     f32x4 wk = {w0, w0, w0, w0};
+    if constexpr (K32) {
+      wk = Mma32<T>::run(za.v, uw32[k * NJ + j], wk);
+    } else {
 #pragma unroll
-    for (int c = 0; c < RC; ++c) wk = Mma16<T>::run(za[c], uw[(k * RC + c) * 4 + j], wk);
+      for (int c = 0; c < RC; ++c) wk = Mma16<T>::run(za.c[c], uw[(k * RC + c) * NJ + j], wk);
+    }
     return wk;
   };
-  auto scatter = [&](const f32x4& wk, const float(&dyf)[4][4], int k, int j, float(&own)[4][4], float(&S)[4]) {
+  auto scatter = [&](const f32x4& wk, const float(&dyf)[4][NJ], int k, int j, float(&own)[4][NJ],
+                     float(&S)[NSC][NJ]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if (i >= k)
-        own[i - k][j] = fmaf(dyf[i][j], wk[i], own[i - k][j]);
+      const int r = i - k;  // dx row of this contribution, relative to 4q
+      if (r >= 0)
+        own[r][j] = fmaf(dyf[i][j], wk[i], own[r][j]);
       else
-        S[j] = fmaf(dyf[i][j], wk[i], S[j]);  // row 4q-1, of the group above
+        S[-r - 1][j] = fmaf(dyf[i][j], wk[i], S[-r - 1][j]);  // row 4q-1-m of the group above
     }
   };
-  float carry[4] = {0.f, 0.f, 0.f, 0.f};  // W 2: group 3's open row of the tile before
-  auto close_rows = [&](const float(&own)[4][4], const float(&S)[4], int tile) {
+  float carry[NSC][NJ];  // group 3's open rows of the tile before
+#pragma unroll
+  for (int i = 0; i < NSC; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) carry[i][j] = 0.f;
+  auto close_rows = [&](const float(&own)[4][NJ], const float(&S)[NSC][NJ], int tile) {
     const int src = ((lane + 16) & 63) << 2;  // ds_bpermute byte index of the group below
     const bool top = q == 3;
+    float recv[NSC][NJ];
+#pragma unroll
+    for (int m = 0; m < NSC; ++m)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        recv[m][j] = W > 1 ? __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(S[m][j]))) : 0.f;
     const int cur_off = tile < tile1 ? dxlane_off + (tile * 16 - rb) * dxrowb : kOobTile;
-    const int prev_off = tile > tile0 ? dxlane_off + ((tile - 1) * 16 - rb) * dxrowb : kOobTile;
+    const int prev_off = tile > tile0 && tile <= tile1 ? dxlane_off + ((tile - 1) * 16 - rb) * dxrowb : kOobTile;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const bool open = W == 2 && i == 3;  // takes the group below's sums
-      float v[4];
+      const bool open = W > 1 && i >= kFirstOpen;  // takes the group below's sums
+      float v[NJ];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < NJ; ++j) {
         v[j] = own[i][j];
-        if (open)
-          v[j] = (top ? carry[j] : v[j]) + __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(S[j])));
+        if (open) v[j] = (top ? carry[i - kFirstOpen][j] : v[j]) + recv[3 - i][j];
       }
-      bstore64<true>(u32x2{pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])}, rdx,
-                     (top && open ? prev_off : cur_off) + i * dxrowb);
+      LV::store(LV::template pack<T>(v), rdx, (top && open ? prev_off : cur_off) + i * dxrowb);
     }
+    if constexpr (W > 1) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) carry[j] = own[3][j];
+      for (int i = 0; i < NSC; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) carry[i][j] = own[kFirstOpen + i][j];
+    }
   };
   auto compute_tile = [&](int it, const TileIn& in) {
     const int tile = tile0 + it;
-    u32x2 zA[RC], zT[RC];
-    in.zr.finish(zA, tile * 16 + n, zr, zrk, Tn, q);
-    // z_eff transposed (rank n, rows 4q..4q+3) through an exact identity product
+    const ZO zA = z_op(in, tile);
+    u32x2 zT[RC];  // z_eff transposed (rank n, rows 4q..4q+3) through an exact identity / selection product
 #pragma unroll
     for (int c = 0; c < RC; ++c) {
-      const f32x4 tz = Mma16<T>::run(zA[c], ident, f32x4{0.f, 0.f, 0.f, 0.f});
+      f32x4 tz;
+      if constexpr (K32)
+        tz = Mma32<T>::run(zA.v, sel[c], f32x4{0.f, 0.f, 0.f, 0.f});
+      else
+        tz = Mma16<T>::run(zA.c[c], ident, f32x4{0.f, 0.f, 0.f, 0.f});
       zT[c] = u32x2{pack2<T>(tz[0], tz[1]), pack2<T>(tz[2], tz[3])};
     }
-    float dyf[4][4], own[4][4], S[4];
+    float dyf[4][NJ], own[4][NJ], S[NSC][NJ];
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        dyf[m][j] = Mma16<T>::to_f(elem16x2(in.dyr[m], j));
-        own[m][j] = S[j] = 0.f;
+      for (int j = 0; j < NJ; ++j) {
+        dyf[m][j] = Mma16<T>::to_f(LV::elem(in.dyr[m], j));
+        own[m][j] = 0.f;
       }
+#pragma unroll
+    for (int m = 0; m < NSC; ++m)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) S[m][j] = 0.f;
     f32x4 dz[RC];
 #pragma unroll
     for (int c = 0; c < RC; ++c) dz[c] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -263,52 +420,78 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
       // the wave barriers keep the compiler from moving an LDS write above
       // another lane's read (the hardware keeps a wavefront's LDS order)
       __builtin_amdgcn_wave_barrier();
+      float gf[4][NJ];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) gf[i][j] = dyf[i][j] * Mma16<T>::to_f(LV::elem(in.xr[i - k + W - 1], j));
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
         scatter(tap_w(zA, k, j, k == 0 ? res : 0.f), dyf, k, j, own, S);
-        float gf[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) gf[i] = dyf[i][j] * Mma16<T>::to_f(elem16x2(in.xr[i - k + W - 1], j));
-        const u32x2 gk = {pack2<T>(gf[0], gf[1]), pack2<T>(gf[2], gf[3])};
+        const u32x2 gk = {pack2<T>(gf[0][j], gf[1][j]), pack2<T>(gf[2][j], gf[3][j])};
         *reinterpret_cast<u32x2*>(my_g + gw_lane + 8 * j) = gk;
 #pragma unroll
         for (int c = 0; c < RC; ++c) du[k][c][j] = Mma16<T>::run(zT[c], gk, du[k][c][j]);
       }
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
+      for (int s2 = 0; s2 < NS; ++s2) {
         const u32x2 lo = lds_read_tr16(my_g + gr_lane + s2 * (8 * 32 + 16));
         const u32x2 hi = lds_read_tr16(my_g + gr_lane + s2 * (8 * 32 + 16) + 32);
         const u32x4 ga = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll
-        for (int c = 0; c < RC; ++c) dz[c] = Mma32<T>::run(ga, my_uz[((k * RC + c) * 2 + s2) * 64 + lane], dz[c]);
+        for (int c = 0; c < RC; ++c) dz[c] = Mma32<T>::run(ga, my_uz[((k * RC + c) * NS + s2) * 64 + lane], dz[c]);
       }
     }
     close_rows(own, S, tile);
-    const int buf = it & 1;
+    const int slot = it % DZB;
+    const int buf = (it / DZB) & 1;
 #pragma unroll
     for (int c = 0; c < RC; ++c)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) dzred[buf][wave][c * 256 + (((4 * q + i) * 16 + n) ^ (q << 4))] = dz[c][i];
-    __syncthreads();
+      for (int i = 0; i < 4; ++i) dzred[buf][rw][cw][slot][c * 256 + (((4 * q + i) * 16 + n) ^ (q << 4))] = dz[c][i];
+    if (slot == DZB - 1 || it == nit - 1) {
+      __syncthreads();
+      // the batch's sums go out at raised wave priority: every wavefront waits
+      // at the next batch's barrier for the slowest one here
+      __builtin_amdgcn_s_setprio(1);
+      constexpr int PER_RUN = RC * 256;
+      constexpr int NTH = 64 * NW;
+      static_assert(DZB * PER_RUN % NTH == 0, "whole passes over a full batch");
 #pragma unroll
-    for (int c = 0; c < RC; ++c) {
-      const int e = (int)threadIdx.x, rr = e >> 4, r = 16 * c + (e & 15);
-      const int pos = c * 256 + (e ^ (((e >> 6) & 3) << 4));
-      float v = dzred[buf][0][pos];
+      for (int ri = 0; ri < NRW; ++ri) {
+        const Run& ru = ri == 0 ? runs[0] : runs[NRW - 1];
+        // rows of run ri from its base row; t >= T falls outside the resource
+        const rsrc_t rout = run_rsrc(part_dz + ((int64_t)cg * a.BT + ru.row0 + ru.rb) * a.dzld, Tn - ru.rb, a.dzld * 4);
+        const int tb = ru.tile0 + it - slot;  // run ri's tile of slot 0
 #pragma unroll
-      for (int w2 = 1; w2 < 4; ++w2) v += dzred[buf][w2][pos];
-      // ranks >= R store nothing (rows past T lie outside the resource)
-      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rpz,
-                                            r < R ? ((tile * 16 + rr - rb) * a.dzld + r) * 4 : kOobLane, 0, 0);
+        for (int m = 0; m < DZB * PER_RUN / NTH; ++m) {
+          const int e2 = (int)threadIdx.x + m * NTH;
+          const int sl = e2 / PER_RUN, rem = e2 - sl * PER_RUN;
+          const int c = rem >> 8, rr = (rem >> 4) & 15, nn = rem & 15;
+          const int r = 16 * c + nn;
+          const int ti = tb + sl;  // the slot's tile of run ri
+          const int pos = rem ^ (((rem >> 6) & 3) << 4);  // as written
+          float v = dzred[buf][ri][0][sl][pos];
+#pragma unroll
+          for (int w2 = 1; w2 < NCW; ++w2) v += dzred[buf][ri][w2][sl][pos];
+          // slots past this batch, tiles past the run and ranks >= R store nothing
+          const bool ok = sl <= slot && ti < ru.tile1 && r < R;
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), rout,
+                                                ok ? ((ti * 16 + rr - ru.rb) * a.dzld + r) * 4 : kOobLane, 0, 0);
+        }
+      }
+      __builtin_amdgcn_s_setprio(0);
     }
   };
 
+  // Every wavefront of the workgroup runs nit iterations (the barriers of the
+  // dz batches are shared); tiles past its own run load and store nothing.
   TileIn ta, tb;
   load_tile(tile0, ta);
   __builtin_amdgcn_sched_barrier(0);  // the first tile's loads go out before the U staging waits
-  stage_uops<W, RC>(uw, my_uz, U, sw, R, RK, D, a.uld, d0, q, n, lane);
-  const int nit = tile1 - tile0;
+  stage_uops<W, RC, NJ, NS, !K32>(uw, my_uz, U, sw, R, RK, D, a.uld, d0, q, n, lane);
+  if constexpr (K32) stage_uw32<W, NJ>(uw32, U, sw, R, RK, D, a.uld, d0, q, n);
   for (int it = 0; it < nit; it += 2) {
     load_tile(tile0 + it + 1, tb);
     __builtin_amdgcn_sched_barrier(0);  // issue the next tile's loads before this tile's waits
@@ -317,22 +500,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
     __builtin_amdgcn_sched_barrier(0);
     if (it + 1 < nit) compute_tile(it + 1, tb);
   }
-  if constexpr (W == 2) {
-    // the tile after the run closes its last row
+  if constexpr (W > 1) {
+    // The tile after the longest run (loaded into the buffer that is next in
+    // turn) closes that run's last rows; in a shorter run it lies past tile1
+    // and stores nothing.
     auto flush = [&](const TileIn& in) {
-      u32x2 zA[RC];
-      in.zr.finish(zA, tile1 * 16 + n, zr, zrk, Tn, q);
-      float dyf[4][4], own[4][4], S[4];
+      const int tile = tile0 + nit;
+      const ZO zA = z_op(in, tile);
+      float dyf[4][NJ], own[4][NJ], S[NSC][NJ];
 #pragma unroll
       for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          dyf[m][j] = Mma16<T>::to_f(elem16x2(in.dyr[m], j));
-          own[m][j] = S[j] = 0.f;
+        for (int j = 0; j < NJ; ++j) {
+          dyf[m][j] = Mma16<T>::to_f(LV::elem(in.dyr[m], j));
+          own[m][j] = 0.f;
         }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) scatter(tap_w(zA, 1, j, 0.f), dyf, 1, j, own, S);
-      close_rows(own, S, tile1);
+      for (int m = 0; m < NSC; ++m)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) S[m][j] = 0.f;
+#pragma unroll
+      for (int k = 1; k < W; ++k)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) scatter(tap_w(zA, k, j, 0.f), dyf, k, j, own, S);
+      close_rows(own, S, tile);
     };
     if (nit & 1)
       flush(tb);
@@ -340,10 +531,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
       flush(ta);
   }
 
-  // ---- dU partial of this run: rows r < RK of U_eff, the wavefront's 64 columns
-  // per tap.  The resource spans the run's RK x W*D partial, so rows r >= RK fall
-  // outside it (the host keeps (RK + 16) * W * D * 4 bytes below kOobLane, so no
-  // offset wraps).
+  if constexpr (NRW == 2) {
+    // The second run's wavefronts hand their dU sums to the first run's
+    // wavefronts of the same chunk through LDS (the dz buffers, now free).
+    float* xch = &dzred[0][0][0][0][0];
+    constexpr int NDU = W * RC * NJ * 4;  // dU floats per lane
+    static_assert(NCW * NDU * 64 <= 2 * NRW * NCW * DZB * RC * 256, "dU exchange fits the dz buffers");
+    __syncthreads();
+    if (rw == 1) {
+#pragma unroll
+      for (int k = 0; k < W; ++k)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) xch[((cw * W + k) * 16 + j * 4 + i) * 64 + lane] = du[k][0][j][i];
+    }
+    __syncthreads();
+    if (rw == 1) return;
+#pragma unroll
+    for (int k = 0; k < W; ++k)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) du[k][0][j][i] += xch[((cw * W + k) * 16 + j * 4 + i) * 64 + lane];
+  }
+
+  // ---- dU partial of this workgroup row: rows r < RK of U_eff, the wavefront's
+  // CPW columns per tap.  The resource spans the RK x W*D partial, so rows r >=
+  // RK fall outside it (the host keeps (RK + 16) * W * D * 4 bytes below
+  // kOobLane, so no offset wraps).
   const rsrc_t rdu = make_rsrc(part_du + (int64_t)du_slot * a.dupr * a.uld, lr_dupart_bytes(RK, a.uld, 0, D));
   const int du_lane = chv ? (4 * q * a.uld + col) * 4 : kOobLane;
 #pragma unroll
@@ -351,10 +567,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 8))) voi
 #pragma unroll
     for (int c = 0; c < RC; ++c)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        bstore128<false>(u32x4{__float_as_uint(du[k][c][0][i]), __float_as_uint(du[k][c][1][i]),
-                               __float_as_uint(du[k][c][2][i]), __float_as_uint(du[k][c][3][i])},
-                         rdu, du_lane + ((16 * c + i) * a.uld + k * D) * 4);
+      for (int i = 0; i < 4; ++i) {
+        const int off = du_lane + ((16 * c + i) * a.uld + k * D) * 4;
+        if constexpr (NJ == 4)
+          bstore128<false>(u32x4{__float_as_uint(du[k][c][0][i]), __float_as_uint(du[k][c][1][i]),
+                                 __float_as_uint(du[k][c][2][i]), __float_as_uint(du[k][c][3][i])},
+                           rdu, off);
+        else
+          __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(du[k][c][0][i]), __float_as_uint(du[k][c][1][i])},
+                                                rdu, off, 0, 0);
+      }
 }
 
 // ------------------------------------------------------------------- host
@@ -417,6 +639,37 @@ inline bool bwd_f32dx_room(const LrProblem& p) {
 }
 inline bool bwd_f32dx(const LrProblem& p) { return !bwd_dx_split(p) && bwd_f32dx_room(p); }
 
+// One-pass problems of one rank chunk (W <= 4), and of two at W 1 and 4, whose x,
+// dy and dx together are more than the last-level cache (256 MB) keeps, with
+// rows of whole 128-byte lines: lr_bwd_mfma's 16-row tiles (at one chunk its loads
+// and stores are whole lines; for lr_bwd_t32 neither cache policies nor a second
+// tile in flight nor other run lengths closed the gap).  bf16, t32 -> 16-row tiles: B4 T8192
+// D2048 R16 W 1 93 -> 74 us, W 2 96 -> 75 (5.4 TB/s), W 4 101 -> 91, R31 + static W 1
+// 98 -> 88, W 4 127 -> 121; B16 T4096 D2048 R16 W 2 184 -> 151; B2 T8192 D4096 R31 +
+// static W 4 125 -> 121.  Below (B4 T4096 D2048, 201 MB) R16 W 2 40 -> 44, W 4
+// 46 -> 54; rows of 6000 bytes (D 3000) R16 W 4 282 -> 319; two chunks at W 2 78 -> 82
+// (B6 T4096 D2048), W 3 equal.  The sizes are one group's, so that a grouped
+// call's results are those of its groups' single calls.
+inline bool bwd_streams(const LrProblem& p) {
+  const int64_t rk = p.R + (p.static_w ? 1 : 0), bytes = 3 * p.B * p.T * p.D * 2;
+  if (rk > 32 || p.W > 4 || p.D % 64 != 0) return false;
+  if (rk <= 16 || p.W == 1) return bytes > 240000000;
+  return p.W == 4 && bytes > 280000000;
+}
+
+// A launch's kernel and workgroups: lr_bwd_t32 (32 channels to a wavefront, rows
+// 32 to a tile), or lr_bwd_mfma (16 rows): two runs to a workgroup and 64
+// channels at one rank chunk, 32 channels at two, 64 at three and four.
+struct BwdShape {
+  bool t32;
+  int rows, cpw, nrw;
+};
+inline BwdShape bwd_shape(const LrProblem& p) {
+  const int rc = bwd_rc(p);
+  if (rc <= 2 && !bwd_streams(p)) return {true, kT32Rows, kT32Chan, 1};
+  return {false, 16, rc == 2 ? 32 : 64, rc == 1 ? 2 : 1};
+}
+
 }  // namespace
 
 // The passes of a backward launch sequence: kernel ranks rofs .. rofs+RK-1 (R
@@ -468,26 +721,26 @@ int64_t lr_bwd_max_run_tiles(const LrProblem& p) {
 
 namespace {
 
-// Tiles per run of lr_bwd_t32: a CU holds one of its workgroups, so a launch
+// Tiles per run: a CU holds one of its workgroups, so a launch
 // takes ceil(workgroups / 256) rounds of a run's length each, and a few
 // workgroups past a round cost as much as a full one (B1 T8192 D768 R15 + static
 // W 8: runs of 3 tiles are 258 workgroups and took 48 us, runs of 4 31 us; B3
 // T4788 D3712 R32: 270 workgroups 163 us, 225 116 us).  Of the run
 // lengths that fill one to eight rounds, the one with the least time by a
 // model: per round a launch's start and end (6 us) and the run's tiles, and
-// every run's dU partial written and read once.  dflt: no such length (more
+// every dU partial (one to nrw runs) written and read once.  dflt: no such length (more
 // sequences than eight rounds hold).
-int64_t t32_run_tiles(const LrProblem& p, int64_t ntile, int64_t cols, int64_t dflt) {
+int64_t bwd_run_tiles(const LrProblem& p, int rows, int nrw, int64_t ntile, int64_t cols, int64_t dflt) {
   constexpr int64_t kCus = 256;
-  const double tile_us = 0.6 * (p.W < 2 ? 2 : p.W > 8 ? 8 : p.W) * (bwd_rc(p) == 2 ? 1.25 : 1.0);
+  const double tile_us = 0.6 * (p.W < 2 ? 2 : p.W > 8 ? 8 : p.W) * (bwd_rc(p) == 2 ? 1.25 : 1.0) * rows / kT32Rows;
   const double part_us = (double)(p.R + (p.static_w ? 1 : 0)) * p.W * p.D * 8 / 5e6;
   int64_t best = dflt;
   double best_us = -1;
   for (int64_t rounds = 1; rounds <= 8; ++rounds) {
-    const int64_t per_seq = rounds * kCus / (p.B * cols);  // runs a sequence may take
+    const int64_t per_seq = rounds * kCus * nrw / (p.B * cols);  // runs a sequence may take
     if (per_seq < 1) continue;
     const int64_t seg = (ntile + per_seq - 1) / per_seq, runs = p.B * ((ntile + seg - 1) / seg);
-    const double us = rounds * (6.0 + seg * tile_us) + runs * part_us;
+    const double us = rounds * (6.0 + seg * tile_us) + (runs + nrw - 1) / nrw * part_us;
     if (best_us < 0 || us < best_us) {
       best = seg;
       best_us = us;
@@ -501,28 +754,27 @@ int64_t t32_run_tiles(const LrProblem& p, int64_t ntile, int64_t cols, int64_t d
 // number of workgroups (and the dU partials nrp times fewer).
 LrBwdArgs make_bwd_args(const LrProblem& p, int target_waves, bool split) {
   LrBwdArgs a;
-  const int rc = bwd_rc(p);
-  const bool t32 = rc <= 2;  // lr_bwd_t32, else lr_bwd_mfma
-  const int cpw = t32 ? kT32Chan : 64, ncw = 256 / cpw, rows = t32 ? kT32Rows : 16;
+  const BwdShape sh = bwd_shape(p);
+  const int rows = sh.rows, ncw = 256 / sh.cpw;
   a.Tn = (int)p.T;
   a.D = (int)p.D;
   a.R = (int)p.R;
   a.RK = (int)p.R + (p.static_w ? 1 : 0);
   a.residual = p.residual;
-  a.nch = (int)((p.D + cpw - 1) / cpw);
+  a.nch = (int)((p.D + sh.cpw - 1) / sh.cpw);
   a.ncg = (a.nch + ncw - 1) / ncw;
   const int64_t ntile = (p.T + rows - 1) / rows;
   a.nrp = split ? bwd_rank_passes(p) : 1;
   const int64_t cap = lr_bwd_max_run_tiles(p) * 16 / rows;  // >= 1 (lr_mfma_ok)
   int64_t seg = (p.B * ntile * a.ncg * ncw * a.nrp + target_waves - 1) / target_waves;
-  if (t32) seg = t32_run_tiles(p, ntile, (int64_t)a.ncg * a.nrp, seg);
+  if (bwd_rc(p) <= 2) seg = bwd_run_tiles(p, rows, sh.nrw, ntile, (int64_t)a.ncg * a.nrp, seg);
   if (seg < 1) seg = 1;
   if (seg > ntile) seg = ntile;
   if (seg > cap) seg = cap;
   a.seg = (int)seg;
   a.nspb = (int)((ntile + seg - 1) / seg);
   a.nseg = (int)(p.B * a.nspb);
-  a.npair = a.nseg;
+  a.npair = (a.nseg + sh.nrw - 1) / sh.nrw;
   a.sp0 = 0;
   a.nblk = a.npair * a.ncg * a.nrp;
   a.BT = p.B * p.T;
@@ -671,7 +923,7 @@ struct BwdWs {
 BwdWs bwd_ws(const LrProblem& p, bool split) {
   const LrBwdArgs a = make_bwd_args(contiguous_problem(p), kBwdTargetWaves, split);
   BwdWs w;
-  w.slots = du_slots(a.nseg, a.seg);
+  w.slots = du_slots(a.npair, a.seg);
   // one dz partial slot per pass of taps (the passes of ranks fill disjoint columns)
   const int64_t dz = (int64_t)npasses((int)p.W, bwd_rc(p)) * a.ncg * a.BT * a.R * 4;
   w.dz_off = 0;
@@ -684,18 +936,19 @@ BwdWs bwd_ws(const LrProblem& p, bool split) {
 
 // One pass's kernel for wq taps and rc rank chunks.
 template <typename T>
-hipError_t dispatch_bwd_kernel(const LrBwdArgs& a, int wq, int rc, bool f32, hipStream_t stream) {
-  if (rc <= 2) return lr_bwd_t32_launch<T>(a, wq, rc, f32, stream);
-  if (f32 || a.accdx || a.nodx) return hipErrorInvalidValue;  // three and four rank chunks take one pass
-  if (rc == 3 && wq == 1)
-    lr_bwd_mfma<T, 1, 3><<<a.nblk, 256, 0, stream>>>(a);
-  else if (rc == 3 && wq == 2)
-    lr_bwd_mfma<T, 2, 3><<<a.nblk, 256, 0, stream>>>(a);
-  else if (rc == 4 && wq == 1)
-    lr_bwd_mfma<T, 1, 4><<<a.nblk, 256, 0, stream>>>(a);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+hipError_t dispatch_bwd_kernel(const LrBwdArgs& a, const BwdShape& sh, int wq, int rc, bool f32, hipStream_t stream) {
+  if (sh.t32) return lr_bwd_t32_launch<T>(a, wq, rc, f32, stream);
+  if (f32 || a.accdx || a.nodx) return hipErrorInvalidValue;  // 16-row tiles take one pass
+#define DC_BWD_CASE(WW, CC, NRW, CPW)                                                        \
+  if (wq == WW && rc == CC) {                                                                \
+    lr_bwd_mfma<T, WW, CC, NRW, CPW><<<a.nblk, 64 * (256 / CPW) * NRW, 0, stream>>>(a);      \
+    return hipGetLastError();                                                                \
+  }
+  DC_BWD_CASE(1, 1, 2, 64) DC_BWD_CASE(2, 1, 2, 64) DC_BWD_CASE(3, 1, 2, 64) DC_BWD_CASE(4, 1, 2, 64)
+  DC_BWD_CASE(1, 2, 1, 32) DC_BWD_CASE(4, 2, 1, 32)
+  DC_BWD_CASE(1, 3, 1, 64) DC_BWD_CASE(2, 3, 1, 64) DC_BWD_CASE(1, 4, 1, 64)
+#undef DC_BWD_CASE
+  return hipErrorInvalidValue;
 }
 
 template <typename T>
@@ -707,6 +960,7 @@ hipError_t launch_bwd(const LrProblem* p, int G) {
   const bool f32 = bwd_f32dx(p[0]), dxs = bwd_dx_split(p[0]);
   LrBwdArgs a = make_bwd_args(p[0], kBwdTargetWaves, dxs);
   const BwdWs w = bwd_ws(p[0], dxs);
+  const BwdShape sh = bwd_shape(p[0]);
   a.xld = (int)p[0].xld();
   a.dxld = (int)p[0].dxld();
   a.yhd = (int)p[0].yhd();
@@ -781,13 +1035,13 @@ hipError_t launch_bwd(const LrProblem* p, int G) {
         for (int g = 0; g < G; ++g)
           b.grp[g].sw = p[g].static_w ? (const void*)((const T*)p[g].static_w + f.kofs * D) : nullptr;
       }
-      if ((e = dispatch_bwd_kernel<T>(b, f.W, rc, f32, p[0].stream)) != hipSuccess) return e;
+      if ((e = dispatch_bwd_kernel<T>(b, sh, f.W, rc, f32, p[0].stream)) != hipSuccess) return e;
     }
     return hipSuccess;
   };
-  DuParts t(a.nseg, w.slots);
+  DuParts t(a.npair, w.slots);
   for (;; t.next()) {
-    a.sp0 = t.run0;
+    a.sp0 = t.run0 * sh.nrw;
     a.npair = t.n;
     a.nblk1 = a.npair * a.ncg * a.nrp;
     a.nblk = G * a.nblk1;
