@@ -262,7 +262,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) voi
   // pre_z rows 8q .. 8q+7 of a tile, the lane's 2 channels (rows past the run read 0)
   auto load_pre = [&](int tile, uint32_t(&pr)[8]) {
     const bool live = chv && tile < tile1;
-    const int toff = (tile - tile0) * 32 * K * 2;
+    const int toff = live ? (tile - tile0) * 32 * K * 2 : 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) pr[i] = bload32(rp, live ? lane_off + toff + i * K * 2 : kProjOob);
   };
@@ -383,10 +383,14 @@ struct ProjBwdPlan {
   int ncg, nrun, seg;
 };
 
+// Longest run (tiles of 32 rows) whose byte offsets stay below kProjOob; >= 4
+// where proj_shape_ok holds.
+int64_t max_run_tiles(const ProjProblem& p) { return (kProjOob - 1) / (32 * p.K * 2); }
+
 // Runs of 32-row tiles: of the run lengths that fill an eighth of the chip's 256
 // workgroups (one to a CU) to four rounds of them, the one with the least time by a model of a
 // round's start, its tiles, and the fp32 dW_in partial each run writes and the
-// reduction reads.
+// reduction reads.  At most max_run_tiles (M 4194304 K 4096 would take runs of 2 GiB).
 ProjBwdPlan bwd_plan(const ProjProblem& p) {
   constexpr int64_t kSlots = 256;
   ProjBwdPlan pl;
@@ -406,6 +410,8 @@ ProjBwdPlan bwd_plan(const ProjProblem& p) {
       best_us = us;
     }
   }
+  const int64_t cap = max_run_tiles(p);
+  if (best > cap) best = cap;
   pl.seg = (int)best;
   pl.nrun = (int)((ntile + best - 1) / best);
   return pl;
@@ -475,10 +481,8 @@ bool proj_shape_ok(const ProjProblem& p) {
   if (N < 1 || N > 128 || p.K % 8 != 0) return false;
   // row indices (tiles of 16, blocks of 64 rows) are int: m0 + 64 stays in range
   if (p.M > INT32_MAX - 64) return false;
-  // byte offsets within int32, below the out-of-range offset
-  if ((int64_t)N * p.K * 4 >= kProjOob || 32 * p.K * 2 >= kProjOob) return false;
-  const ProjBwdPlan pl = bwd_plan(p);
-  return (int64_t)(pl.seg + 3) * 32 * p.K * 2 < kProjOob;
+  // byte offsets within int32, below the out-of-range offset (runs of four tiles at least: K <= 8.3 M)
+  return N * p.K * 4 < kProjOob && max_run_tiles(p) >= 4;
 }
 
 int64_t proj_bwd_ws_bytes(const ProjProblem& p) {
