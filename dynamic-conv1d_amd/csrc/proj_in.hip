@@ -374,43 +374,226 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) voi
     }
 }
 
+// The backward on 16-row x 64-channel tiles: a row group's 16 lanes load and store
+// whole 128-byte lines, past the caches (nontemporal).  proj_bwd's 64-byte pieces
+// keep half as many bytes in flight to HBM (2.7 TB/s at M 65536 K 2048 N 45, this one
+// 4.7; what the two request is equal by count), but its tiles halve the products and the
+// staging, and its default-policy loads hit where pre_z is still in the last-level
+// cache.  Which one runs: line_tiles.
+template <typename T, int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) void proj_bwd_lines(ProjArgs a) {
+  constexpr int NP = NB * 16;          // ranks padded to whole 16-rank chunks (zero past N)
+  constexpr int N32 = (NP + 31) / 32;  // 32-rank steps of the dpre_z product
+  constexpr int NP32 = N32 * 32;       // ranks of the row-major dz tile (zero past N)
+  constexpr int DROW = NP32 * 2 + 16;  // bytes per row of the row-major dz tile (16-byte pad)
+  constexpr int TROW = 16 * 2 + 8;     // bytes per rank of the rank-major tile (8-byte pad)
+  __shared__ __attribute__((aligned(16))) uint8_t dzr[2][16 * DROW];  // [row][rank]
+  __shared__ __attribute__((aligned(16))) uint8_t dzt[2][NP * TROW];  // [rank][row]
+
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int q = lane >> 4, n = lane & 15;
+  const int blk = xcd_remap(blockIdx.x, a.nblk);
+  const int cg = blk % a.ncg, run = blk / a.ncg;
+  const int M = a.M, K = a.K, N = a.N, R = a.R;
+  const int col = cg * 256 + wave * 64 + 4 * n;  // the lane's first channel (K % 8 == 0: all four in or out)
+  const bool chv = col < K;
+  const int ntile = (M + 15) >> 4;
+  const int tile0 = run * a.seg, tile1 = min(tile0 + a.seg, ntile);
+  const int r0 = tile0 * 16;
+  const int nrow = max(min(M - r0, (tile1 - tile0) * 16), 0);
+  const rsrc_t rp = make_rsrc_wave<kProjOob>(a.pre + (int64_t)min(r0, M) * K, (int64_t)nrow * K * 2);
+  const rsrc_t rd = make_rsrc_wave<kProjOob>(a.dpre + (int64_t)min(r0, M) * K, (int64_t)nrow * K * 2);
+  const int lane_off = (4 * q * K + col) * 2;  // the lane's row-4q channels; lanes past K take kProjOob alone
+
+  // W_in operands of the dpre_z product, as proj_bwd's, for four channels
+  u32x4 wop[N32][4];
+  {
+    const rsrc_t rw = make_rsrc_wave<kProjOob>(a.w, (int64_t)N * K * 2);
+#pragma unroll
+    for (int s = 0; s < N32; ++s) {
+      u32x2 rows8[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int c = 32 * s + 8 * q + e;
+        rows8[e] = bload64(rw, chv && c < N ? (c * K + col) * 2 : kProjOob);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          wop[s][j][h] = elem16x2(rows8[2 * h], j) | (elem16x2(rows8[2 * h + 1], j) << 16);
+    }
+  }
+  f32x4 dw[NB][4];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dw[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // dz tile staging: NP32 x 16 elements; rank c is group c / R, rank c % R, zero past N and past M
+  constexpr int SPT = (NP32 * 16 + 255) / 256;
+  uint32_t sv[SPT];
+  auto load_dz = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < SPT; ++i) {
+      const int e = i * 256 + (int)threadIdx.x;
+      const int row = e / NP32, c = e - row * NP32;
+      const int m = tile * 16 + row;
+      // an unconditional load from a valid address (group 0's first element when
+      // the element lies outside the tile), so no load sits under a branch
+      const bool ok = e < NP32 * 16 && c < N && m < M && tile < tile1;
+      const int g = ok ? c / R : 0;
+      const uint16_t* src = ok ? pick4(a.dz, g) + ((int64_t)m * R + (c - g * R)) : a.dz[0];
+      const uint32_t v = *src;
+      sv[i] = ok ? v : 0u;
+    }
+  };
+  auto store_dz = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < SPT; ++i) {
+      const int e = i * 256 + (int)threadIdx.x;
+      if (e >= NP32 * 16) break;
+      const int row = e / NP32, c = e - row * NP32;
+      *reinterpret_cast<uint16_t*>(&dzr[b][row * DROW + c * 2]) = (uint16_t)sv[i];
+      if (c < NP) *reinterpret_cast<uint16_t*>(&dzt[b][c * TROW + row * 2]) = (uint16_t)sv[i];
+    }
+  };
+  // pre_z rows 4q .. 4q+3 of a tile, the lane's 4 channels (rows past the run read 0)
+  auto load_pre = [&](int tile, u32x2(&pr)[4]) {
+    const bool live = chv && tile < tile1;
+    const int toff = live ? (tile - tile0) * 16 * K * 2 : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pr[i] = bload64<kNt>(rp, live ? lane_off + toff + i * K * 2 : kProjOob);
+  };
+
+  u32x2 pa[4], pb[4];
+  load_dz(tile0);
+  store_dz(0);
+  load_pre(tile0, pa);
+  __syncthreads();
+  auto compute = [&](int tile, int b, const u32x2(&pr)[4]) {
+    // dpre_z = dz W_in: A = dz row n, ranks 32s + 8q .. +7
+    f32x4 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < N32; ++s) {
+      const u32x4 ar = *reinterpret_cast<const u32x4*>(&dzr[b][n * DROW + (32 * s + 8 * q) * 2]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[j] = Mma32<T>::run(ar, wop[s][j], acc[j]);
+    }
+    const int toff = (tile - tile0) * 16 * K * 2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      bstore64<true>(u32x2{pack2<T>(acc[0][i], acc[1][i]), pack2<T>(acc[2][i], acc[3][i])}, rd,
+                     chv ? lane_off + toff + i * K * 2 : kProjOob);
+    // dW_in += dz^T pre_z: A = dz^T (ranks 16c + n, rows 4q .. 4q+3), B = pre_z rows 4q .. 4q+3 of channel col + j
+    u32x2 bop[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      bop[j][0] = elem16x2(pr[0], j) | (elem16x2(pr[1], j) << 16);
+      bop[j][1] = elem16x2(pr[2], j) | (elem16x2(pr[3], j) << 16);
+    }
+#pragma unroll
+    for (int c = 0; c < NB; ++c) {
+      const u32x2 at = *reinterpret_cast<const u32x2*>(&dzt[b][(16 * c + n) * TROW + 8 * q]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) dw[c][j] = Mma16<T>::run(at, bop[j], dw[c][j]);
+    }
+  };
+
+  const int nt = tile1 - tile0;
+  for (int it = 0; it < nt; it += 2) {
+    // tile it from (buffer 0, pa); tile it + 1 from (buffer 1, pb)
+    load_dz(tile0 + it + 1);
+    load_pre(tile0 + it + 1, pb);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(tile0 + it, 0, pa);
+    store_dz(1);  // buffer 1 was last read before the previous barrier
+    __syncthreads();
+    if (it + 1 >= nt) break;  // uniform across the workgroup
+    load_dz(tile0 + it + 2);
+    load_pre(tile0 + it + 2, pa);
+    __builtin_amdgcn_sched_barrier(0);
+    compute(tile0 + it + 1, 1, pb);
+    store_dz(0);
+    __syncthreads();
+  }
+
+  // dW_in partial of this run: rank 16c + 4q + i, channels col .. col+3
+  const rsrc_t rpart = make_rsrc_wave<kProjOob>(a.part + (int64_t)run * N * K, (int64_t)N * K * 4);
+#pragma unroll
+  for (int c = 0; c < NB; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int rk = 16 * c + 4 * q + i;
+      bstore128<false>(u32x4{__float_as_uint(dw[c][0][i]), __float_as_uint(dw[c][1][i]), __float_as_uint(dw[c][2][i]),
+                             __float_as_uint(dw[c][3][i])},
+                       rpart, chv && rk < N ? (rk * K + col) * 4 : kProjOob);
+    }
+}
+
 // ------------------------------------------------------------------ host
 namespace {
 
 int nb_of(int64_t N) { return (int)((N + 15) / 16); }
 
 struct ProjBwdPlan {
+  bool lines;  // proj_bwd_lines (16-row tiles), else proj_bwd (32)
   int ncg, nrun, seg;
 };
 
-// Longest run (tiles of 32 rows) whose byte offsets stay below kProjOob; >= 4
-// where proj_shape_ok holds.
-int64_t max_run_tiles(const ProjProblem& p) { return (kProjOob - 1) / (32 * p.K * 2); }
+// proj_bwd_lines where pre_z comes from HBM and the products are few: ranks N <= 64
+// from 64 MB of pre_z and dpre_z on, N <= 96 where they are more than the
+// last-level cache (256 MB) can hold a part of; more ranks are bound by products.
+// bf16, proj_bwd -> proj_bwd_lines, inputs not in the cache (and in it, from the
+// call before): M 16384 K 2048 N 15 48 -> 32 us (30 -> 31), K 4096 N 63 108 -> 63
+// (61 -> 64), N 45 104 -> 66 (62 -> 66), M 65536 K 2048 N 45 185 -> 115, M 32768 K
+// 4096 N 93 199 -> 166; below: M 8192 K 1024 N 45 23 -> 25 (19 -> 25), M 16384 K
+// 4096 N 93 110 -> 105 (70 -> 105), N 127 122 -> 162.  And in the smallest problems,
+// which are a launch's start and end: M 512 K 512 N 15 9.4 -> 8.9 us (8.1 -> 7.2), M
+// 2048 K 512 N 15 10.1 -> 9.7 (9.1 -> 8.7); N 45 12.3 -> 14.0 (12.2 -> 14.1).
+bool line_tiles(const ProjProblem& p) {
+  const int64_t N = p.G * p.R, bytes = p.M * p.K * 4;
+  if (N <= 64) return bytes > 64000000 || p.M * p.K * N <= (20 << 20);
+  return N <= 96 && bytes > 400000000;
+}
 
-// Runs of 32-row tiles: of the run lengths that fill an eighth of the chip's 256
+// Longest run (tiles of `rows` rows) whose byte offsets stay below kProjOob; >= 4
+// where proj_shape_ok holds.
+int64_t max_run_tiles(const ProjProblem& p, int rows) { return (kProjOob - 1) / (rows * p.K * 2); }
+
+// Runs of tiles.  proj_bwd: of the run lengths that fill an eighth of the chip's 256
 // workgroups (one to a CU) to four rounds of them, the one with the least time by a model of a
 // round's start, its tiles, and the fp32 dW_in partial each run writes and the
-// reduction reads.  At most max_run_tiles (M 4194304 K 4096 would take runs of 2 GiB).
+// reduction reads.  proj_bwd_lines: two workgroups to a CU, one round.  Either way
+// at most max_run_tiles (M 4194304 K 4096 would take runs of 2 GiB).
 ProjBwdPlan bwd_plan(const ProjProblem& p) {
   constexpr int64_t kSlots = 256;
   ProjBwdPlan pl;
-  const int64_t ntile = (p.M + 31) / 32;
+  pl.lines = line_tiles(p);
+  const int rows = pl.lines ? 16 : 32;
+  const int64_t ntile = (p.M + rows - 1) / rows, cap = max_run_tiles(p, rows);
   pl.ncg = (int)((p.K + 255) / 256);
-  const double tile_us = 1.2, part_us = (double)p.G * p.R * p.K * 8 / 5e6;
   int64_t best = ntile;
-  double best_us = -1;
-  for (int64_t slots = kSlots / 8; slots <= 4 * kSlots; slots *= 2) {
-    const int64_t runs = slots / pl.ncg;
-    if (runs < 1) continue;
-    const int64_t seg = (ntile + runs - 1) / runs, nrun = (ntile + seg - 1) / seg;
-    const double rounds = slots <= kSlots ? 1 : (double)slots / kSlots;
-    const double us = rounds * (4.0 + seg * tile_us) + nrun * part_us;
-    if (best_us < 0 || us < best_us) {
-      best = seg;
-      best_us = us;
+  if (pl.lines) {
+    const int64_t runs = 2 * kSlots / pl.ncg;
+    if (runs > 1) best = (ntile + runs - 1) / runs;
+  } else {
+    const double tile_us = 1.2, part_us = (double)p.G * p.R * p.K * 8 / 5e6;
+    double best_us = -1;
+    for (int64_t slots = kSlots / 8; slots <= 4 * kSlots; slots *= 2) {
+      const int64_t runs = slots / pl.ncg;
+      if (runs < 1) continue;
+      const int64_t seg = (ntile + runs - 1) / runs, nrun = (ntile + seg - 1) / seg;
+      const double rounds = slots <= kSlots ? 1 : (double)slots / kSlots;
+      const double us = rounds * (4.0 + seg * tile_us) + nrun * part_us;
+      if (best_us < 0 || us < best_us) {
+        best = seg;
+        best_us = us;
+      }
     }
   }
-  const int64_t cap = max_run_tiles(p);
   if (best > cap) best = cap;
   pl.seg = (int)best;
   pl.nrun = (int)((ntile + best - 1) / best);
@@ -458,7 +641,11 @@ hipError_t launch_bwd(const ProjProblem& p) {
   a.ncg = pl.ncg;
   a.seg = pl.seg;
   a.nblk = pl.ncg * pl.nrun;
-  switch (nb_of(a.N) * 8 + (int)p.G) {
+  switch (pl.lines ? nb_of(a.N) : nb_of(a.N) * 8 + (int)p.G) {  // 1 .. 6 (line_tiles), or 9 .. 68
+#define DC_PL(NBV) \
+  case NBV: proj_bwd_lines<T, NBV><<<a.nblk, 256, 0, p.stream>>>(a); break;
+    DC_PL(1) DC_PL(2) DC_PL(3) DC_PL(4) DC_PL(5) DC_PL(6)
+#undef DC_PL
 #define DC_PB(NBV, NGV) \
   case NBV * 8 + NGV: proj_bwd<T, NBV, NGV><<<a.nblk, 512, 0, p.stream>>>(a); break;
 #define DC_PBG(NBV) DC_PB(NBV, 1) DC_PB(NBV, 2) DC_PB(NBV, 3) DC_PB(NBV, 4)
@@ -482,7 +669,7 @@ bool proj_shape_ok(const ProjProblem& p) {
   // row indices (tiles of 16, blocks of 64 rows) are int: m0 + 64 stays in range
   if (p.M > INT32_MAX - 64) return false;
   // byte offsets within int32, below the out-of-range offset (runs of four tiles at least: K <= 8.3 M)
-  return N * p.K * 4 < kProjOob && max_run_tiles(p) >= 4;
+  return N * p.K * 4 < kProjOob && max_run_tiles(p, 32) >= 4;
 }
 
 int64_t proj_bwd_ws_bytes(const ProjProblem& p) {
