@@ -618,17 +618,17 @@ inline int bwd_rank_passes(const LrProblem& p) {
 // R73 + static W2, 3 passes, against 0.02 + 2%).
 constexpr int kBwdMaxBf16DxPasses = 4;
 constexpr int kBwdMaxBf16DxRankPasses = 2;
-// Passes of ranks with dy in [B, T, D] whose dx fits one launch
-// (lr_dx_split_shape: W <= 8 up to kernel rank 64, W 5 / 4 up to 96 / 128) or,
-// with dy in either layout, two (W 9-16 up to 64, over the fp32 accumulator): the
+// Passes of ranks whose dx fits one launch
+// (lr_dx_split_shape: W <= 8 up to kernel rank 64, W 5 / 4 up to 96 / 128) or
+// two (W 9-16 up to 64, over the fp32 accumulator), with dy in either layout: the
 // passes form dz and dU only (DXM 3) and lr_dx_t32 forms dx over all ranks and
 // taps in one launch, rounded once (no fp32 accumulator).  Passes of taps alone
 // (two rank chunks above W 4) keep dx: split off it measured 160 -> 166 us at B4
 // T4096 D2048 R31 + static W 8.
 inline bool bwd_dx_split(const LrProblem& p) {
   const int64_t hd = p.yhd();
-  // head-major dy: two launches only, where a chunk's heads fit one resource
-  const bool dy_ok = hd == p.D || (lr_dx_two_passes(p.W) && (127 / hd + 2) * (p.T + 64) * hd * 2 < kMaxSeqBytes);
+  // head-major dy: where a 128-channel chunk lies in one head, or its heads fit one resource
+  const bool dy_ok = hd == p.D || hd % 128 == 0 || (127 / hd + 2) * (p.T + 64) * hd * 2 < kMaxSeqBytes;
   return bwd_rank_split(p) && lr_dx_split_shape(p.R + (p.static_w ? 1 : 0), p.W) && dy_ok;
 }
 // The workspace keeps room for the accumulator whether or not dx is split off:

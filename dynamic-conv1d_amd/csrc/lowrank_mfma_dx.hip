@@ -49,7 +49,7 @@ static hipError_t dx_taps(const LrProblem* p, int G, const void* const* z, int z
   a.nch = (int)((p0.D + 127) / 128);
   a.zld = zld;
   a.xld = (int)p0.D;       // dy: [B, T, D],
-  a.zrp = (int)p0.yhd();   // with M also head-major
+  a.zrp = (int)p0.yhd();   // or head-major
   a.yhd = (int)p0.dxld();  // dx rows
   a.uld = p0.uld();
   // runs as the forward's, capped so that the rows of dy, dx and z a run

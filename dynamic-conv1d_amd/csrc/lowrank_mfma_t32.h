@@ -303,10 +303,15 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) 
   if (sg >= a.nseg) return;
   const T32Run run(a, sg);
   const int rb = run.rb, tile0 = run.tile0, tile1 = run.tile1, ntile = (Tn + 31) >> 5;
-  // dy is [B, T, D] (hd == D), with M also head-major [B, D/hd, T, hd]: the resource then
+  // dy is [B, T, D] (hd == D) or head-major [B, D/hd, T, hd]: the resource then
   // spans the chunk's heads (loads check the row against T)
-  const int hd = M ? a.zrp : a.xld, yh = M ? dl / hd : 0, yh0 = M ? chunk * 128 / hd : 0;
-  const int yhl = M ? min(chunk * 128 + 127, D - 1) / hd : 0;
+  const int hd = a.zrp;
+  int yh = 0, yh0 = 0, yhl = 0;
+  if (hd != D) {  // the divisions take 0.4 us
+    yh = dl / hd;
+    yh0 = chunk * 128 / hd;
+    yhl = min(chunk * 128 + 127, D - 1) / hd;
+  }
   const int dyrowb = hd * 2, dxrowb = a.yhd * 2, zld = a.zld;
   const rsrc_t rdy = run_rsrc(dy + run.row0 * a.xld + ((int64_t)yh0 * Tn + rb) * hd,
                               (int64_t)(yhl - yh0) * Tn + Tn - rb, dyrowb);
@@ -342,7 +347,7 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) 
     u32x4 dyr[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      dyr[i] = bload128(rdy, M && tile * 32 + 8 * q + i >= Tn ? kOobTile : dylane + toff + i * dyrowb);
+      dyr[i] = bload128(rdy, tile * 32 + 8 * q + i >= Tn ? kOobTile : dylane + toff + i * dyrowb);
     u32x4 zc[2][NC];
 #pragma unroll
     for (int h = 0; h < 2; ++h)

@@ -231,7 +231,8 @@ int64_t dc_lowrank_bwd_grouped_ws_bytes(int64_t G, int64_t B, int64_t T, int64_t
  * when dy_hd = 0 and head-major [B, D/dy_hd, T, dy_hd] otherwise (the layout
  * of dc_lowrank_fwd_grouped's y_hd).  dstatic_w is NULL exactly when static_w
  * is.  Per group, results are bitwise those of dc_lowrank_bwd (with a head
- * dim: when it is a multiple of 64, else the generic kernels; dU and dstatic_w
+ * dim: when it is a multiple of 64, else the generic kernels, and dx at kernel
+ * ranks 33 .. 128 when it is a multiple of 128 or T * dy_hd < 2^26; dU and dstatic_w
  * to their sums' last bits where rows of x or dx are so far apart that a run of
  * rows has to be shorter than the contiguous call's).  Replaces
  * README.md:57-110's three backwards (lowrank.py:251-299 each) and the
