@@ -242,7 +242,13 @@ struct GroupedModuleFn : public Function<GroupedModuleFn> {
       dys.push_back(grad_in(grads[g], x.scalar_type()));
       dyp.p[g] = ptr(dys.back());
     }
-    Tensor dx = at::empty({s.B, s.T, C}, x.options()), dpre = at::empty_like(pre), dw = at::empty_like(w_in);
+    // pre_z or proj_in.weight wanted (inputs 1, 2): a frozen projection has no backward
+    const bool proj = ctx->needs_input_grad(1) || ctx->needs_input_grad(2);
+    Tensor dx = at::empty({s.B, s.T, C}, x.options()), dpre, dw;
+    if (proj) {
+      dpre = at::empty_like(pre);
+      dw = at::empty_like(w_in);
+    }
     Tensor dU = at::empty_like(U), dsw = at::empty_like(sw);
     const Tensor dz = z_buffer(x, s);
     const auto it = ctx->saved_data.find("zeff");
@@ -250,7 +256,7 @@ struct GroupedModuleFn : public Function<GroupedModuleFn> {
     const int64_t nz = zeff.defined() ? abi.lowrank_zeff_bytes(s.B, s.T, s.D, s.R, s.W, s.dt, 1) : 0;
     const int64_t n1 = abi.lowrank_bwd_grouped_ws_bytes(s.G, s.B, s.T, s.D, s.R, s.W, s.dt, 1);
     check(n1, "grouped lowrank backward workspace query");
-    const int64_t n2 = abi.proj_in_bwd_ws_bytes(s.G, s.B * s.T, s.K, s.R, s.dt);
+    const int64_t n2 = proj ? abi.proj_in_bwd_ws_bytes(s.G, s.B * s.T, s.K, s.R, s.dt) : 0;
     check(n2, "proj_in backward workspace query");
     // one workspace: proj_in's backward runs after the convolutions' on the same stream
     const Tensor ws = bytes_like(x, std::max<int64_t>(std::max(n1, n2), 1));
@@ -261,9 +267,10 @@ struct GroupedModuleFn : public Function<GroupedModuleFn> {
                                   zeff.defined() ? ze.in() : nullptr, nz, dyp.in(), hd, ptr(dx), C, dzs.out(),
                                   dUs.out(), dsws.out(), ptr(ws), n1, s.B, s.T, s.D, s.R, s.W, s.dt, 1, st),
           "grouped lowrank backward");
-    check(abi.proj_in_bwd(ptr(pre), ptr(w_in), dzs.in(), ptr(dpre), ptr(dw), ptr(ws), n2, s.G, s.B * s.T, s.K, s.R, s.dt,
-                          st),
-          "proj_in backward");
+    if (proj)
+      check(abi.proj_in_bwd(ptr(pre), ptr(w_in), dzs.in(), ptr(dpre), ptr(dw), ptr(ws), n2, s.G, s.B * s.T, s.K, s.R,
+                            s.dt, st),
+            "proj_in backward");
     return {dx, dpre, dw, dU, dsw, Tensor()};
   }
 };
