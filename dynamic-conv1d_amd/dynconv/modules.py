@@ -166,8 +166,8 @@ class GroupedLowRankDynamicShortConvolution(nn.Module):
         # _module_proj_in: nothing else may be looking at the projection
         if (_capi.binding is not None and _plain_linear(self.proj_in)
                 and not torch.is_autocast_enabled(pre_z.device.type)):
-            ys = _capi.binding.grouped_module(x, pre_z, self.proj_in.weight, self.proj_out, self.proj_out_bias,
-                                              self.head_dim)
+            hd = None if self.head_dim is None else int(self.head_dim)  # as the Python path takes it
+            ys = _capi.binding.grouped_module(x, pre_z, self.proj_in.weight, self.proj_out, self.proj_out_bias, hd)
             if ys is not None:
                 return ys
         zs = list(_module_proj_in(self.proj_in, pre_z, G, R))  # one GEMM for every group
