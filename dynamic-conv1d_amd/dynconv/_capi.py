@@ -10,6 +10,7 @@ import ctypes
 import functools
 import os
 import threading
+import warnings
 
 import torch
 
@@ -55,7 +56,7 @@ _lib = None
 _lock = threading.Lock()
 # The native autograd binding (csrc/torch_binding.cpp, built beside the library),
 # once load() has given it the library; None before that, or where it was not
-# built for this torch: the Functions in headwise.py, lowrank.py and modules.py
+# built, or for another torch (with a warning): the Functions in headwise.py, lowrank.py and modules.py
 # take every call then, as they take each call that the binding declines.
 binding = None
 
@@ -63,12 +64,20 @@ binding = None
 def _load_binding(path: str):
     try:
         from . import _binding as b
-    except ImportError:
+    except ModuleNotFoundError:  # not built
+        return None
+    except ImportError as e:
+        warnings.warn(f"dynconv/_binding.so does not load ({e}): {_SLOW}", stacklevel=3)
         return None
     if b.torch_version != torch.__version__:
+        warnings.warn(f"dynconv/_binding.so was built for torch {b.torch_version}, not {torch.__version__}: {_SLOW}",
+                      stacklevel=3)
         return None
     b.init(path)
     return b
+
+
+_SLOW = "the Python autograd Functions take every call, at about twice the host time (rebuild with build.py)"
 
 
 def load(path: str = LIB_PATH):
