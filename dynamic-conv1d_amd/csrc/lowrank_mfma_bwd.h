@@ -34,7 +34,7 @@ struct LrBwdArgs {
   int xld;    // row stride of x (elements)
   int dxld;   // row stride of dx (elements; the fp32 accumulator's D past four passes)
   int dxsld;  // row stride of dx for the last pass over the accumulator (DXM 2)
-  int nodx;   // dz and dU only (DXM 3): a separate launch (lr_dx_mfma) forms dx over all ranks
+  int nodx;   // dz and dU only (DXM 3): launches of their own (lr_dx_t32) form dx over all ranks
   int nrp;    // with nodx: passes of 32 ranks in this launch (R and RK are then the problem's), else 1
   // z rows: zld elements apart, ranks < zr loaded, ranks zr .. zrk-1 of z_eff
   // added as the static rank (ZRaw).  z itself (zld = zr = R, zrk = RK) when

@@ -728,8 +728,10 @@ namespace {
 // T4788 D3712 R32: 270 workgroups 163 us, 225 116 us).  Of the run
 // lengths that fill one to eight rounds, the one with the least time by a
 // model: per round a launch's start and end (6 us) and the run's tiles, and
-// every dU partial (one to nrw runs) written and read once.  dflt: no such length (more
-// sequences than eight rounds hold).
+// every dU partial (one to nrw runs) written and read once.  The plan is one group's: a
+// grouped launch has G times the workgroups, but its results are to be those of its
+// groups' single calls, and so are its workspace shares.  dflt: no such length
+// (more sequences than eight rounds hold).
 int64_t bwd_run_tiles(const LrProblem& p, int rows, int nrw, int64_t ntile, int64_t cols, int64_t dflt) {
   constexpr int64_t kCus = 256;
   const double tile_us = 0.6 * (p.W < 2 ? 2 : p.W > 8 ? 8 : p.W) * (bwd_rc(p) == 2 ? 1.25 : 1.0) * rows / kT32Rows;

@@ -1,4 +1,6 @@
-// Lowrank backward on gfx950 matrix cores, one and two rank chunks (bf16 / fp16).
+// Lowrank backward on gfx950 matrix cores, one and two rank chunks (bf16 / fp16):
+// every pass of a problem that takes several, and one-pass problems up to the size of
+// the last-level cache (larger ones: bwd_streams in lowrank_mfma_bwd.hip).
 //
 // One pass over x and dy produces dx, dz, dU and dstatic_w (reference:
 // lowrank.py:87-140 and 159-205, two kernels that both read dy).
@@ -48,8 +50,8 @@
 // first tile).
 //
 // A tile's rows are loaded into the registers of one whose rows have just been
-// converted to fp32, so one tile (two at one rank chunk and W <= 4, NBUF) is in
-// flight while one is computed.
+// converted to fp32, so one tile is in flight while one is computed (a second one in
+// flight at W <= 4: B4 T4096 D2048 R16 W 2 40 -> 42 us, B8 T8192 D4096 equal).
 //
 // dz partial sums over the 256 channels are added in LDS in wave order, once
 // per DZB tiles, and written as one fp32 partial per 256-channel group; dU
@@ -82,10 +84,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   constexpr int NO = W > 1 ? W - 1 : 1;     // open rows of a group (none at W 1)
   constexpr int kFirstOpen = 9 - W;         // rows kFirstOpen .. 7 take the group below's sums
   constexpr bool NODX = DXM == 3;
-  // U operands in registers where they fit beside two tiles (one rank chunk, W <= 4), else in LDS
+  // U operands in registers where they fit (one rank chunk, W <= 4), else in LDS
   constexpr bool UREG = RC == 1 && W <= 4;
-  // tiles in flight while one is computed: two where the registers hold them
-  constexpr int NBUF = 1;
   constexpr int DZB = RC == 1 ? 2 : 1;      // tiles per dz batch
   constexpr int GPL = 272;                  // bytes per 4-row plane of the G tile (32 channels x 8 B + 16)
   typedef Pair LV;
@@ -187,8 +187,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     u32x4 z32[RC == 2 ? 2 : 1];
     typename DV::type dxo[ACC && DXO == kDxoAhead ? 8 : 1];
   };
-  TileIn in[NBUF];
-  auto load_tile = [&](TileIn& in, int tile) {
+  TileIn in;
+  auto load_tile = [&](int tile) {
     const int xtoff = tile < tile1 ? (tile * 32 - rb - kofs) * xrowb : kOobTile;
     const bool ylive = NODX ? tile < tile1 : tile <= tile1;
     const int toff = ylive ? (tile * 32 - rb) * rowb : kOobTile;
@@ -206,8 +206,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
     if constexpr (ACC && DXO == kDxoAhead) load_dxo(tile, in.dxo);
   };
-#pragma unroll
-  for (int i = 0; i < NBUF; ++i) load_tile(in[i], tile0 + i);
+  load_tile(tile0);
   // HX: x rows 8q-W+1 .. 8q-1 are own rows of the lane group above (lane - 16),
   // or for group 0 those of group 3 in the tile before (prev: loaded for the run's
   // first tile), passed with one ds_bpermute each.
@@ -339,7 +338,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     u32x4 v;     // two: ranks 8q..8q+7
   };
   // the tile's z operands of half h, from the loaded registers
-  auto z_op = [&](const TileIn& in, int tile, int h) {
+  auto z_op = [&](int tile, int h) {
     ZA o;
     if constexpr (RC == 2)
       o.v = in.z32[h];
@@ -423,7 +422,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
 
   const int nit = tile1 - tile0;
-  auto do_tile = [&](int it, TileIn& in) {
+  auto do_tile = [&](int it) {
     const int tile = tile0 + it;
     float xf[NR][2], dyf[8][2];
     const int above = ((lane + 48) & 63) << 2;  // ds_bpermute byte index of lane - 16
@@ -444,7 +443,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int m = 0; m < 8; ++m)
 #pragma unroll
       for (int j = 0; j < 2; ++j) dyf[m][j] = Mma16<T>::to_f(LV::elem(in.dyr[m], j));
-    ZA zA[2] = {z_op(in, tile, 0), z_op(in, tile, 1)};
+    ZA zA[2] = {z_op(tile, 0), z_op(tile, 1)};
     __builtin_amdgcn_sched_barrier(0);
     typename DV::type dxo[ACC ? 8 : 1] = {};
     if constexpr (ACC && DXO == kDxoTile) load_dxo(tile, dxo);
@@ -452,7 +451,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
       for (int i = 0; i < 8; ++i) dxo[i] = in.dxo[DXO == kDxoAhead ? i : 0];
     }
-    load_tile(in, tile + NBUF);
+    load_tile(tile + 1);
     __builtin_amdgcn_sched_barrier(0);  // the next tile's loads go out before this tile's products
 
     // z_eff transposed (rank n, rows 8q..8q+7): exact identity / selection products
@@ -544,8 +543,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       static_assert(DZB * RC * 512 == 2 * 512, "one pair of ranks per thread");
       const int e2 = 2 * (int)threadIdx.x;
       const int sl = e2 / (RC * 512), rem = e2 - sl * (RC * 512);
-      const int c = rem >> 9, in = rem & 511, rr = in >> 4, r = 16 * c + (in & 15);
-      const int pos = c * 512 + (in ^ (((in >> 7) & 3) << 4));
+      const int c = rem >> 9, el = rem & 511, rr = el >> 4, r = 16 * c + (el & 15);
+      const int pos = c * 512 + (el ^ (((el >> 7) & 3) << 4));
       f32x2 v = *reinterpret_cast<const f32x2*>(&dzred[buf][sl][0][pos]);
 #pragma unroll
       for (int w2 = 1; w2 < NW; ++w2) {
@@ -561,20 +560,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       __builtin_amdgcn_s_setprio(0);
     }
   };
-  for (int it = 0; it < nit; it += NBUF) {
-    do_tile(it, in[0]);
-    if constexpr (NBUF == 2)
-      if (it + 1 < nit) do_tile(it + 1, in[1]);
-  }
+  for (int it = 0; it < nit; ++it) do_tile(it);
   if constexpr (!NODX && W > 1) {
     // The tile after the run (loaded) closes its last rows: rows 0 .. W-2 only.
-    const bool second = NBUF == 2 && (nit & 1);  // the buffer that holds it
     float dyf[8][2], own[8][2], S[NO][2];
 #pragma unroll
     for (int m = 0; m < 8; ++m) {
-      const uint32_t v = second ? in[NBUF - 1].dyr[m] : in[0].dyr[m];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) dyf[m][j] = Mma16<T>::to_f(LV::elem(v, j));
+      for (int j = 0; j < 2; ++j) dyf[m][j] = Mma16<T>::to_f(LV::elem(in.dyr[m], j));
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) own[i][0] = own[i][1] = 0.f;
@@ -582,12 +575,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int i = 0; i < NO; ++i) S[i][0] = S[i][1] = 0.f;
 #pragma unroll
     for (int h = 0; h < (W <= 5 ? 1 : 2); ++h) {
-      ZA za = z_op(in[0], tile1, h);
-      if constexpr (NBUF == 2) {
-        const ZA z1 = z_op(in[1], tile1, h);
-        za.c[0][0] = second ? z1.c[0][0] : za.c[0][0];
-        za.c[0][1] = second ? z1.c[0][1] : za.c[0][1];
-      }
+      const ZA za = z_op(tile1, h);
 #pragma unroll
       for (int k = 1; k < W; ++k)
 #pragma unroll
@@ -617,7 +605,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 template <typename T, int W, int RC>
 hipError_t lr_bwd_t32_one(const LrBwdArgs& a, bool f32, hipStream_t stream) {
   if constexpr (RC == 2) {
-    if (a.nodx) {  // dz and dU only (lr_dx_mfma forms dx)
+    if (a.nodx) {  // dz and dU only (lr_dx_t32 forms dx)
       lr_bwd_t32<T, W, RC, false, 3><<<a.nblk, 512, 0, stream>>>(a);
       return hipGetLastError();
     }

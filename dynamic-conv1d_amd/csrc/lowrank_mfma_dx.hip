@@ -1,8 +1,10 @@
-// dx of the lowrank backward over all kernel ranks and taps in one launch
-// (lr_dx_t32, lowrank_mfma_t32.h), for the problems whose backward runs as passes
-// of 32 ranks (lr_bwd_rank_split): those passes then form dz and dU only (lr_bwd_t32's
-// DXM 3), and dx is rounded once, where passes that each added their share rounded
-// it after every pass (or went through an fp32 accumulator).
+// dx of the lowrank backward over all kernel ranks (lr_dx_t32, lowrank_mfma_t32.h),
+// for the problems whose backward runs as passes of 32 ranks (lr_bwd_rank_split):
+// those passes then form dz and dU only (lr_bwd_t32's DXM 3), and dx is rounded
+// once.  Up to W 8 one launch takes all taps; at W 9-16 (kernel rank 33-64) two
+// launches of half the taps each, over an fp32 accumulator that the first stores
+// and the second adds, where the passes themselves would add to it once per
+// 32 ranks and 4 taps.
 #include "lowrank_mfma_t32.h"
 
 namespace dc {

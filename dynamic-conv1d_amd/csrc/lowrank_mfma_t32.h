@@ -14,11 +14,15 @@
 // time (a 16x16x16 product takes as long as a 16x16x32 one).  Channels are
 // computed a pair at a time: 16 accumulators and the pair's fp32 rows are live,
 // the packed results replace the pair's raw rows.
-// B4 T4096 D2048 bf16, before (16 ranks to a product) and now: forward R31 +
-// static 39.1 -> 31.7 us (4.3 TB/s of its bytes), W 8 48 -> 41, R63 + static 47.4 ->
-// 40.4, W 8 80 -> 55, B2 T8192 D4096 R31 + static 63.8 -> 58.8; R32 without the z_eff
-// writer equal.  Backward with this dx launch: R63 + static 166 -> 148, W 8 399 ->
-// 252, R127 + static 322 -> 245.
+// 60-133 VGPRs at 32 ranks, 74-248 at 64 (dx 88-256), none spilled.
+// B4 T4096 D2048 bf16, before (16 ranks to a product) and now, z_eff writer
+// included: forward R31 + static 36.4 -> 29.6 us (4.6 TB/s of its bytes), W 8 38.4 ->
+// 32.8, R63 + static 41.5 -> 36.4, W 8 67 -> 41.7, B2 T8192 D4096 R31 + static 59.4 ->
+// 55.4.  Without the writer R32 and R31 + static at W 3-4 are 1-5% slower at the first
+// size, faster at others (B8 T4096 D4096 W 4 112.5 -> 107.8).  Backward with this dx
+// launch: R63 + static 154 -> 125, W 8 384 -> 233, R127 + static 292 -> 207.
+// What bounds the forward: memory at W 4 (4.6 TB/s, 5.1 for a plain copy of the same
+// tensors); at W 8 the products alone would take 13 of the 33 us (1.35 PFLOP/s).
 #pragma once
 
 #include "lowrank_mfma_fwd_kernel.h"
@@ -126,7 +130,7 @@ struct T32Run {
 // Ends the work on one channel pair: its packed results exist here, and the LDS
 // reads of the next pair's operands come after (a sched_barrier alone does not
 // order pure arithmetic, and the pairs' weights, rows and sums then live together:
-// 256 registers and up to 1.2 KB of spills where one pair at a time takes 130).
+// 256 registers and up to 1.2 KB of spills, against 142 and none at W 4 and 64 ranks).
 __device__ __forceinline__ void end_pair(u32x4 (&o)[8], int h4) {
   asm volatile("" : "+v"(o[0][h4]), "+v"(o[1][h4]), "+v"(o[2][h4]), "+v"(o[3][h4]), "+v"(o[4][h4]), "+v"(o[5][h4]),
                "+v"(o[6][h4]), "+v"(o[7][h4]) : : "memory");
@@ -275,7 +279,7 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_fwd_t32(LrArgs a)
 // rows kofs earlier) adds it and stores dx, rounded once; dx's last kofs rows, which
 // get no terms of M 2's taps, are left to the caller.  Against passes of 32 ranks x 4
 // taps that each added dx into the accumulator, whole backward at B4 T4096 D2048
-// bf16: R40 W 12 616 -> 382 us, R64 W 16 890 -> 534 us.
+// bf16: R40 W 12 530 -> 386 us, R64 W 16 772 -> 534 us.
 template <typename T, int W, int NC, int M = 0>
 __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) {
   constexpr int NWV = t32_wg_waves(W, NC);
