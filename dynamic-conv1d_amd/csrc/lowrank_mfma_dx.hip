@@ -12,8 +12,11 @@ namespace dc {
 template <typename T>
 hipError_t lr_dx_t32_launch(const LrArgs& a, int W, int NC, int M, hipStream_t s) {
 #define DC_DX_CASE(WW, CC)                                                          \
-  if (W == WW && NC == CC && M == 0) {                                                        \
-    lr_dx_t32<T, WW, CC><<<a.nblk, 64 * t32_wg_waves(WW, CC), 0, s>>>(a);           \
+  if (W == WW && NC == CC && M == 0) {                                              \
+    if (a.zrp == a.xld)                                                             \
+      lr_dx_t32<T, WW, CC><<<a.nblk, 64 * t32_wg_waves(WW, CC), 0, s>>>(a);         \
+    else                                                                            \
+      lr_dx_t32<T, WW, CC, 0, true><<<a.nblk, 64 * t32_wg_waves(WW, CC), 0, s>>>(a);\
     return hipGetLastError();                                                       \
   }
   // W x NC <= 16: up to 128 KiB of staged operands (lr_dx_split_shape)

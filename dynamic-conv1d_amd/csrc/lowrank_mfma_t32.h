@@ -280,7 +280,7 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_fwd_t32(LrArgs a)
 // get no terms of M 2's taps, are left to the caller.  Against passes of 32 ranks x 4
 // taps that each added dx into the accumulator, whole backward at B4 T4096 D2048
 // bf16: R40 W 12 530 -> 386 us, R64 W 16 772 -> 534 us.
-template <typename T, int W, int NC, int M = 0>
+template <typename T, int W, int NC, int M = 0, bool HM = M != 0>
 __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) {
   constexpr int NWV = t32_wg_waves(W, NC);
   constexpr int NO = W > 1 ? W - 1 : 1;  // open rows of a group (none at W 1)
@@ -307,15 +307,10 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) 
   if (sg >= a.nseg) return;
   const T32Run run(a, sg);
   const int rb = run.rb, tile0 = run.tile0, tile1 = run.tile1, ntile = (Tn + 31) >> 5;
-  // dy is [B, T, D] (hd == D) or head-major [B, D/hd, T, hd]: the resource then
-  // spans the chunk's heads (loads check the row against T)
-  const int hd = a.zrp;
-  int yh = 0, yh0 = 0, yhl = 0;
-  if (hd != D) {  // the divisions take 0.4 us
-    yh = dl / hd;
-    yh0 = chunk * 128 / hd;
-    yhl = min(chunk * 128 + 127, D - 1) / hd;
-  }
+  // dy is [B, T, D] (hd == D) or, with HM, head-major [B, D/hd, T, hd]: the resource
+  // then spans the chunk's heads (loads check the row against T)
+  const int hd = HM ? a.zrp : a.xld, yh = HM ? dl / hd : 0, yh0 = HM ? chunk * 128 / hd : 0;
+  const int yhl = HM ? min(chunk * 128 + 127, D - 1) / hd : 0;
   const int dyrowb = hd * 2, dxrowb = a.yhd * 2, zld = a.zld;
   const rsrc_t rdy = run_rsrc(dy + run.row0 * a.xld + ((int64_t)yh0 * Tn + rb) * hd,
                               (int64_t)(yhl - yh0) * Tn + Tn - rb, dyrowb);
@@ -351,7 +346,7 @@ __global__ __launch_bounds__(64 * t32_wg_waves(W, NC)) void lr_dx_t32(LrArgs a) 
     u32x4 dyr[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      dyr[i] = bload128(rdy, tile * 32 + 8 * q + i >= Tn ? kOobTile : dylane + toff + i * dyrowb);
+      dyr[i] = bload128(rdy, HM && tile * 32 + 8 * q + i >= Tn ? kOobTile : dylane + toff + i * dyrowb);
     u32x4 zc[2][NC];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
