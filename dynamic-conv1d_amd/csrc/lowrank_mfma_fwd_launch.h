@@ -99,7 +99,7 @@ hipError_t launch_fwd(const LrProblem* p, int G) {
     const int64_t cap = lr_fwd_max_run_tiles(p[0]) / 2, ntile = (p[0].T + 31) / 32;
     if ((zal || a.R % 8 == 7) && a.zrp % 8 == 0 && cap >= 1) {
       const int nwv = t32_wg_waves(W, RC / 2);
-      int64_t seg = t32_run_tiles(p[0].B * ntile * a.nch);
+      int64_t seg = t32_fwd_run_tiles(p[0].B, ntile, (int64_t)G * a.nch, W, RC / 2);
       seg = seg > cap ? cap : seg;
       a.zvec = zal;
       a.seg = (int)(seg > ntile ? ntile : seg);

@@ -29,8 +29,8 @@
 
 namespace dc {
 
-// Tiles per run: 2048 wavefronts where the problem has that many tiles, runs of
-// about 4 tiles above, at most 4096 wavefronts (see fwd_target_waves).
+// Tiles per run of the dx launch: 2048 wavefronts where the problem has that many
+// tiles, runs of about 4 tiles above, at most 4096 wavefronts (see fwd_target_waves).
 inline int64_t t32_run_tiles(int64_t tiles) {
   int64_t w = tiles / 4;
   w = w < 2048 ? (tiles < 2048 ? tiles : 2048) : w > 4096 ? 4096 : w;
@@ -39,6 +39,43 @@ inline int64_t t32_run_tiles(int64_t tiles) {
 
 // Wavefronts per workgroup: as fwd_wg_waves (one workgroup per CU above 80 KiB of operands).
 constexpr int t32_wg_waves(int W, int NC) { return W * NC > 10 ? 8 : 4; }
+
+// Tiles per run of the forward: the length with the least time by a model of
+// workgroups on 256 CUs, fitted at W x NC = 4, 8 and 16 to 84 sweeps of the run
+// length (its choice is within 0.3% of the best length's time on average, 4% at
+// most).  A CU works off k workgroups, each its start (staging of U; part) and its
+// wavefronts' tiles (tile); or, with few of them, the serial chain of a round (lat
+// per tile).  Runs of about 4 tiles whatever the rounds left 2.6 workgroups to a CU
+// at B3 T4788 D3712: bf16 R32 W 4 55.2 -> 48 us, R63 + static W 4 77.4 -> 60.5; B4
+// T6144 D2048 R63 + static W 8 89.9 -> 72.5, B2 T4096 D3072 R32 W 4 31.4 -> 25.5, B4
+// T4096 D2048 equal (31.5).  A grouped call's workgroups count together; y does not
+// depend on the runs.
+inline int64_t t32_fwd_run_tiles(int64_t B, int64_t ntile, int64_t cols, int W, int NC) {
+  struct Cost { double part, tile, lat, start; };
+  constexpr Cost c4{0.46, 0.66, 4.4, 1.4}, c8{4.0, 0.91, 5.0, 9.0}, c16{7.2, 0.86, 8.8, 1.3};
+  const int n = W * NC, nwv = t32_wg_waves(W, NC);
+  const Cost &lo = n <= 8 ? c4 : c8, &hi = n <= 8 ? c8 : c16;
+  const double f = n <= 4 ? 0 : n <= 8 ? (n - 4) / 4.0 : (n - 8) / 8.0;
+  const auto mix = [f](double a, double b) { return a + f * (b - a); };
+  const Cost c{mix(lo.part, hi.part), mix(lo.tile, hi.tile), mix(lo.lat, hi.lat), mix(lo.start, hi.start)};
+  // bound by memory (n <= 4): more workgroups to a CU (B8 T4096 D4096 R31 + static W 4,
+  // runs of 4, 8 and 16 tiles: 104.8, 106.3, 113.4 us)
+  const int64_t longest = n <= 4 ? 4 : 64;
+  const int64_t res = 256 * (n <= 5 ? 4 : 20 / n);  // workgroups resident at once (8 n KiB of 160 each)
+  int64_t best = 1;
+  double best_us = -1;
+  for (int64_t seg = 1; seg <= ntile && seg <= longest; seg += seg < 16 ? 1 : seg / 4) {
+    const int64_t runs = B * ((ntile + seg - 1) / seg), wg = (runs + nwv - 1) / nwv * cols;
+    const double work = (double)((wg + 255) / 256) * (c.part + seg * nwv * c.tile);
+    const double chain = (double)((wg + res - 1) / res) * (seg * c.lat + c.start);
+    const double us = work > chain ? work : chain;
+    if (best_us < 0 || us < best_us) {
+      best = seg;
+      best_us = us;
+    }
+  }
+  return best;
+}
 
 // ub[((k*NC + c)*8 + j)*64 + lane] = U_eff[32c + 8q .. +7, k*D + dl + j], packed
 // (row R is static_w, rows past RK zero; loads as in stage_u).
