@@ -643,11 +643,12 @@ inline bool bwd_f32dx(const LrProblem& p) { return !bwd_dx_split(p) && bwd_f32dx
 // dy and dx together are more than the last-level cache (256 MB) keeps, with
 // rows of whole 128-byte lines: lr_bwd_mfma's 16-row tiles (at one chunk its loads
 // and stores are whole lines; for lr_bwd_t32 neither cache policies nor a second
-// tile in flight nor other run lengths closed the gap).  bf16, t32 -> 16-row tiles: B4 T8192
-// D2048 R16 W 1 93 -> 74 us, W 2 96 -> 75 (5.4 TB/s), W 4 101 -> 91, R31 + static W 1
-// 98 -> 88, W 4 127 -> 121; B16 T4096 D2048 R16 W 2 184 -> 151; B2 T8192 D4096 R31 +
-// static W 4 125 -> 121.  Below (B4 T4096 D2048, 201 MB) R16 W 2 40 -> 44, W 4
-// 46 -> 54; rows of 6000 bytes (D 3000) R16 W 4 282 -> 319; two chunks at W 2 78 -> 82
+// tile in flight nor other run lengths closed the gap).  bf16, t32 -> 16-row tiles, inputs
+// partly left in the cache (and out of it): B4 T8192 D2048 R16 W 1 93 -> 74 us (95 -> 83),
+// W 2 96 -> 75 (97 -> 82), W 4 101 -> 91 (102 -> 97), R31 + static W 1 98 -> 88 (99 -> 92),
+// W 4 127 -> 121 (119 -> 117); B16 T4096 D2048 R16 W 2 184 -> 151; B2 T8192 D4096 R31 +
+// static W 4 125 -> 121 (116 -> 115).  Below, B4 T4096 D2048 (201 MB): R16 W 2 40 -> 44
+// (51 -> 46), W 4 46 -> 54 (57 -> 58), and B3 T5000 D2560 R16 W 2 46 -> 80 (64 -> 87); rows of 6000 bytes (D 3000) R16 W 4 282 -> 319; two chunks at W 2 78 -> 82
 // (B6 T4096 D2048), W 3 equal.  The sizes are one group's, so that a grouped
 // call's results are those of its groups' single calls.
 inline bool bwd_streams(const LrProblem& p) {

@@ -33,16 +33,18 @@
 // takes K = 32 rows per MFMA, twice the rate of K = 16; the dU accumulators of
 // 32 channels take half the registers of 64; and the scatter form, whose sums
 // reach one group up, serves W <= 8.
-// Measured, B4 T4096 D2048 bf16, whole backward before (16-row tiles) and now:
-// W 8 R15 + static 89 -> 81 us, W 16 R16 179 -> 170 us, R63 + static 162 -> 153 us
-// (the two passes of ranks as one launch); W 4 R16 60.7 -> 60.1 us and B2 T8192
-// D4096 R31 + static 124 -> 126 us (equal within the runs); B2 T512 D256 R15 +
-// static 16.6 -> 12.0 us (a launch's serial start, below).  W 4 R16 streams its
-// rows at 5.2 TB/s in the tile loop (38 of 53 us: what bounds it is the memory);
-// two rank chunks are bound by issue: 296 vector and 52 matrix instructions and
-// 42 KB of LDS traffic per tile at two wavefronts per SIMD.  Transposing G with
-// identity products instead of LDS took two rank chunks to 140 us (issue), a
-// second tile in flight changed nothing.
+// Measured, B4 T4096 D2048 bf16, whole backward, inputs out of the cache, 16-row tiles
+// -> these: W 8 R15 + static 82.7 -> 78.0 us, W 16 R16 174 -> 168, W 2 R31 + static 58.6
+// -> 55.3, R63 + static 156 -> 140 (the two passes of ranks as one launch); W 4 R16 56.9
+// -> 56.1 and R31 + static 67.6 -> 67.8 (equal; inputs left in the cache 53 -> 46 and 67
+// -> 63); B2 T512 D256 R15 + static 16.9 -> 13.5 (a launch's serial start, below); R16 at
+// W 1 and 2 44.8 -> 49.3 and 45.8 -> 51.1 (left in the cache equal and 43 -> 40).
+// What bounds it: the chain of one tile (loads, conversions, products, the LDS
+// transposes, sums), which two wavefronts per SIMD overlap in part.  W 4 R16 waits for
+// 28% of its wavefronts' cycles and issues for 39%, W 4 with two rank chunks 37% and 33%,
+// passes that add to dx 43% and 29%, passes of ranks without dx 50% and 29%; the matrix
+// pipe is busy for 13-19%.  Transposing G with identity products instead of LDS took two
+// rank chunks to 140 us, a second tile in flight changed nothing.
 //
 // The launch's start is kept short, since a small problem is little else: the
 // group's pointers are scalar loads at a run-time offset, and the U operands are
@@ -97,11 +99,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // tile's fp32 rows, and take them before the last tap; the fp32 accumulator's at W <=
   // 2 come with the tile, which is too short to hide them, at W 3 at its start.  And the
   // passes that stream more than the last-level cache keeps (an fp32 accumulator, or
-  // two rank chunks at W 4) read dy and store dx nontemporal.  B4 T4096 D2048, rows
-  // held from the tile's start with the open ones carried (8-12 registers spilled),
-  // and now: R31 + static W 8 153 -> 145 us, W 12 226 -> 213, W 20 513 -> 451, R64 W 20
-  // 1115 -> 946, R127 + static W 8 932 -> 815, R160 W 1 379 -> 367, R255 + static W 4
-  // 916 -> 789.  Rows with the tile at W 4 spill (W 20: 788).
+  // two rank chunks at W 4) read dy and store dx nontemporal.  B4 T4096 D2048, inputs
+  // out of the cache, rows held from the tile's start with the open ones carried (8-12
+  // registers spilled) -> now: R31 + static W 8 155 -> 149 us, W 12 227 -> 215, W 20 515
+  // -> 453, R64 W 20 1113 -> 947, R127 + static W 8 934 -> 813, R160 W 1 380 -> 372, R255 +
+  // static W 4 919 -> 794.  Rows with the tile at W 4 spill (W 20: 788).
   enum { kDxoTile, kDxoLastTap, kDxoAhead };
   constexpr int DXO = RC == 1 || DXM == 0 || W == 4 ? kDxoLastTap : W <= 2 ? kDxoAhead : kDxoTile;
   constexpr bool NTP = RC == 2 && (DXM == 1 || DXM == 2 || (ACC && W == 4));

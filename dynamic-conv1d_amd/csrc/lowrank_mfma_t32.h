@@ -15,14 +15,16 @@
 // computed a pair at a time: 16 accumulators and the pair's fp32 rows are live,
 // the packed results replace the pair's raw rows.
 // 60-133 VGPRs at 32 ranks, 74-248 at 64 (dx 88-256), none spilled.
-// B4 T4096 D2048 bf16, before (16 ranks to a product) and now, z_eff writer
-// included: forward R31 + static 36.4 -> 29.6 us (4.6 TB/s of its bytes), W 8 38.4 ->
-// 32.8, R63 + static 41.5 -> 36.4, W 8 67 -> 41.7, B2 T8192 D4096 R31 + static 59.4 ->
-// 55.4.  Without the writer R32 and R31 + static at W 3-4 are 1-5% slower at the first
-// size, faster at others (B8 T4096 D4096 W 4 112.5 -> 107.8).  Backward with this dx
-// launch: R63 + static 154 -> 125, W 8 384 -> 233, R127 + static 292 -> 207.
-// What bounds the forward: memory at W 4 (4.6 TB/s, 5.1 for a plain copy of the same
-// tensors); at W 8 the products alone would take 13 of the 33 us (1.35 PFLOP/s).
+// B4 T4096 D2048 bf16, inputs out of the cache, 16 ranks to a product -> this one,
+// z_eff writer included: forward R31 + static 36.8 -> 30.6 us (4.5 TB/s of its
+// bytes), W 8 47.0 -> 38.7, R63 + static 41.9 -> 37.3, W 8 73.8 -> 51.5, B2 T8192
+// D4096 R31 + static 59.8 -> 56.0.  Without the writer (R32; inference) W 3-4 are 2-6%
+// slower here (R32 30.1 -> 31.5) and 3-7% at B2 T10000 D1536, B3 T4788 D3712 and B6 T2048
+// D4096, faster elsewhere (B12 T4096 D2048 107 -> 85, B2 T2048 D1024 21.6 -> 8.5).
+// Backward with this dx launch: R63 + static 156 -> 140, W 8 390 -> 244, R127 + static
+// 294 -> 244.
+// What bounds the forward: at W 4 the wait for its rows (37% of the wavefronts' cycles;
+// a plain copy of the same tensors reaches 5.1 TB/s); at W 8 issue (44%, 38% vector).
 #pragma once
 
 #include "lowrank_mfma_fwd_kernel.h"
